@@ -134,66 +134,35 @@ __device__ __forceinline__ Wg xcd_grouped() {
   return {t % gx, t / gx, L % 8u + 8u * (rest / G)};
 }
 
-// Sizes are compile-time constants of the generated kernel (batch, M, K, N, and
-// for SPLIT the number of K chunks and their length, a multiple of 16). The
-// workgroup's z index `zid` enumerates batches, or for SPLIT (batch, chunk)
-// pairs, and each SPLIT workgroup stores its raw
-// partial tile to the workspace at ((chunk·batch + b)·M + row)·N + col; a
-// second kernel (gemm_splitk_reduce) sums the chunks in order and applies the
-// epilogue. MODE_C needs C % 4 == 0 and MODE_R needs R % 4 == 0 (R, C: the
-// operand's extents), and both need every other stride a multiple of 4, so a
-// 128-bit load is aligned and either wholly inside the operand or wholly out.
-template <int TM, int TN, int BK, int PF, int AMODE, int BMODE, bool SPLIT, class AV, class BV, class Epi, int WN = 2,
-          bool PRIO = false, int KW = 1, class Args = TcmiArgs>
-__device__ __forceinline__ void gemm_f32(const Args& A, const float* __restrict__ a_ptr,
-                                         const float* __restrict__ b_ptr, const uint32_t batch, const uint32_t M,
-                                         const uint32_t K, const uint32_t N, const uint32_t chunks,
-                                         const uint32_t chunkK, const uint32_t zid, const uint32_t tx,
-                                         const uint32_t ty) {
-  // KW groups of 2 x WN wavefronts; in each group a wavefront owns (TM·16) x (TN·16)
-  // of the BM x BN tile, and group g sums its own part of K (see below).
-  static_assert(KW == 1 || KW == 2 || KW == 4, "K groups");
-  constexpr int THREADS = 64 * 2 * WN;   // threads of one K group
+// A staged tile's padded row stride and floats: As[row][k] or (MODE_R) As[k][row], Bs[k][col]
+// or (MODE_R) Bs[col][k].
+template <int BM, int BN, int BK, int AMODE, int BMODE>
+struct GemmTiles {
+  static constexpr bool A_KMAJOR = AMODE == MODE_R, B_NMAJOR = BMODE == MODE_R;
+  static constexpr int AS = A_KMAJOR ? BM + 4 : BK + 4;
+  static constexpr int BS = B_NMAJOR ? BK + 4 : BN + 4;
+  static constexpr int A = (A_KMAJOR ? BK : BM) * AS, B = (B_NMAJOR ? BN : BK) * BS;
+};
+
+// The BM x BN tile of C at (m0, n0) summed over K in [kbeg, kbeg + slices·BK), elements at or
+// past kend counting as 0, by 2 x WN wavefronts through the LDS buffers As (two A tiles) and Bs
+// (two B tiles): each wavefront's TM x TN accumulators.
+template <int TM, int TN, int BK, int PF, int AMODE, int BMODE, class AV, class BV, int WN, bool PRIO>
+__device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_, const float* __restrict__ Ab,
+                                             const float* __restrict__ Bb, const uint32_t M, const uint32_t N,
+                                             const uint32_t kbeg, const uint32_t kend, const uint32_t slices,
+                                             const uint32_t m0, const uint32_t n0, const int tid, f4 (&acc)[TM][TN]) {
+  constexpr int THREADS = 64 * 2 * WN;
   constexpr int BM = 2 * TM * 16;
   constexpr int BN = WN * TN * 16;
   static_assert(BK == 16 || BK == 32 || BK == 64, "slice depth");
   static_assert(PF == 1 || PF == 2, "prefetch depth");
-  constexpr bool A_KMAJOR = AMODE == MODE_R;   // As[k][row] instead of As[row][k]
-  constexpr bool B_NMAJOR = BMODE == MODE_R;   // Bs[col][k] instead of Bs[k][col]
-  constexpr int AS = A_KMAJOR ? BM + 4 : BK + 4;   // padded row stride of the A tile
-  constexpr int BS = B_NMAJOR ? BK + 4 : BN + 4;   // padded row stride of the B tile
-  // The tiles (and the K groups' hand-over area) live in one LDS pool of this size: two
-  // instantiations of the same size in one kernel (members of one batched launch whose
-  // operand views differ) share it instead of adding up.
-  constexpr int A_TILE = (A_KMAJOR ? BK : BM) * AS, B_TILE = (B_NMAJOR ? BN : BK) * BS;
-  constexpr int TILES = KW * 2 * (A_TILE + B_TILE);
-  float* const pool = lds_pool<TILES + (KW > 1 ? (KW - 1) * THREADS * TM * TN * 4 : 0)>();
-  float (*As_)[2][A_TILE] = reinterpret_cast<float (*)[2][A_TILE]>(pool);
-  float (*Bs_)[2][B_TILE] = reinterpret_cast<float (*)[2][B_TILE]>(pool + KW * 2 * A_TILE);
+  using Tiles = GemmTiles<BM, BN, BK, AMODE, BMODE>;
+  constexpr bool A_KMAJOR = Tiles::A_KMAJOR, B_NMAJOR = Tiles::B_NMAJOR;
+  constexpr int AS = Tiles::AS, BS = Tiles::BS;
+  float (*As)[Tiles::A] = reinterpret_cast<float (*)[Tiles::A]>(As_);
+  float (*Bs)[Tiles::B] = reinterpret_cast<float (*)[Tiles::B]>(Bs_);
 
-  // zid: the workgroup's z index within this launch (blockIdx.z, or its part
-  // below the member index in a batched launch); (tx, ty): its output tile's column
-  // and row (blockIdx.x and .y, or their XCD-grouped places).
-  const uint32_t kz = SPLIT ? zid % chunks : 0u;
-  const uint32_t bz = SPLIT ? zid / chunks : zid;
-  const uint32_t kbeg0 = SPLIT ? kz * chunkK : 0u;
-  const uint32_t kend0 = SPLIT ? min(K, kbeg0 + chunkK) : K;
-  // K groups (KW > 1, for few-tile products: more wavefronts in flight per CU): group g
-  // sums K range [kbeg0 + g·sub, kbeg0 + (g+1)·sub) of this workgroup's range, every
-  // group the same number of slices (a short last range is zero-filled, so every
-  // barrier is reached by all), and the groups' sums are added in order g = 0, 1, ...
-  // after the loop. The split depends on (M, N, K, KW) alone, as everything else here.
-  const int kg = KW == 1 ? 0 : static_cast<int>(threadIdx.x) / THREADS;
-  const uint32_t sub = KW == 1 ? kend0 - kbeg0 : ((kend0 - kbeg0 + KW * BK - 1) / (KW * BK)) * BK;
-  const uint32_t kbeg = kbeg0 + kg * sub;
-  const uint32_t kend = min(kend0, kbeg + sub);
-  float (*As)[A_TILE] = As_[kg];
-  float (*Bs)[B_TILE] = Bs_[kg];
-  const uint32_t m0 = ty * BM, n0 = tx * BN;
-  const float* __restrict__ Ab = a_ptr + AV::batch(bz);
-  const float* __restrict__ Bb = b_ptr + BV::batch(bz);
-
-  const int tid = KW == 1 ? static_cast<int>(threadIdx.x) : static_cast<int>(threadIdx.x) % THREADS;
   const int lane = tid & 63;
   const int wave = tid >> 6;
   const int wm = wave / WN, wn = wave % WN;
@@ -340,7 +309,6 @@ __device__ __forceinline__ void gemm_f32(const Args& A, const float* __restrict_
     }
   };
 
-  f4 acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -391,7 +359,6 @@ __device__ __forceinline__ void gemm_f32(const Args& A, const float* __restrict_
     if (PRIO) __builtin_amdgcn_s_setprio(0);
   };
 
-  const uint32_t slices = KW == 1 ? (kend - kbeg + BK - 1) / BK : sub / BK;
   load_slice(st0, kbeg);
   store_slice(st0, 0);
   if (PF == 2 && slices > 1) load_slice(st1, kbeg + BK);
@@ -419,6 +386,116 @@ __device__ __forceinline__ void gemm_f32(const Args& A, const float* __restrict_
       __syncthreads();
     }
   }
+}
+
+// The accumulators stored: lane (t16, q) of tile (i, j) holds row t16, columns 4q .. 4q+3 of
+// it; row0 and first are this lane's row and first column in tile (0, 0). SPLIT stores the
+// raw sums of chunk kz to the workspace, otherwise the epilogue runs on each element.
+template <int TM, int TN, bool SPLIT, class Epi, class Args>
+__device__ __forceinline__ void gemm_store(const Args& A, const f4 (&acc)[TM][TN], const uint32_t batch, const uint32_t M,
+                                           const uint32_t N, const uint32_t kz, const uint32_t bz, const uint32_t row0,
+                                           const uint32_t first) {
+  constexpr bool VOUT = true;
+  if (SPLIT) {
+    float* __restrict__ part = A.ws + (size_t)(kz * batch + bz) * M * N;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const uint32_t row = row0 + i * 16;
+        const uint32_t col0 = first + j * 16;
+        if (row >= M) continue;
+        if (N % 4 == 0 && VOUT) {
+          if (col0 < N) *reinterpret_cast<f4*>(part + (size_t)row * N + col0) = acc[i][j];
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (col0 + r < N) part[(size_t)row * N + col0 + r] = acc[i][j][r];
+        }
+      }
+    return;
+  }
+  // Epilogue: the fused body on each accumulator element, then the store.
+  const Epi epi;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const uint32_t row = row0 + i * 16;
+      const uint32_t col0 = first + j * 16;
+      if (row >= M) continue;
+      const uint32_t o = (bz * M + row) * N + col0;
+      if (N % 4 == 0 && VOUT) {
+        if (col0 < N) {
+          f4 v;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = epi(A, o + r, acc[i][j][r]);
+          *reinterpret_cast<f4*>(A.out + o) = v;
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (col0 + r < N) A.out[o + r] = epi(A, o + r, acc[i][j][r]);
+      }
+    }
+  }
+}
+
+// Sizes are compile-time constants of the generated kernel (batch, M, K, N, and
+// for SPLIT the number of K chunks and their length, a multiple of 16). The
+// workgroup's z index `zid` enumerates batches, or for SPLIT (batch, chunk)
+// pairs, and each SPLIT workgroup stores its raw
+// partial tile to the workspace at ((chunk·batch + b)·M + row)·N + col; a
+// second kernel (gemm_splitk_reduce) sums the chunks in order and applies the
+// epilogue. MODE_C needs C % 4 == 0 and MODE_R needs R % 4 == 0 (R, C: the
+// operand's extents), and both need every other stride a multiple of 4, so a
+// 128-bit load is aligned and either wholly inside the operand or wholly out.
+template <int TM, int TN, int BK, int PF, int AMODE, int BMODE, bool SPLIT, class AV, class BV, class Epi, int WN = 2,
+          bool PRIO = false, int KW = 1, class Args = TcmiArgs>
+__device__ __forceinline__ void gemm_f32(const Args& A, const float* __restrict__ a_ptr,
+                                         const float* __restrict__ b_ptr, const uint32_t batch, const uint32_t M,
+                                         const uint32_t K, const uint32_t N, const uint32_t chunks,
+                                         const uint32_t chunkK, const uint32_t zid, const uint32_t tx,
+                                         const uint32_t ty) {
+  // KW groups of 2 x WN wavefronts; in each group a wavefront owns (TM·16) x (TN·16)
+  // of the BM x BN tile, and group g sums its own part of K (see below).
+  static_assert(KW == 1 || KW == 2 || KW == 4, "K groups");
+  constexpr int THREADS = 64 * 2 * WN;   // threads of one K group
+  constexpr int BM = 2 * TM * 16;
+  constexpr int BN = WN * TN * 16;
+  using Tiles = GemmTiles<BM, BN, BK, AMODE, BMODE>;
+  // The tiles (and the K groups' hand-over area) live in one LDS pool of this size: two
+  // instantiations of the same size in one kernel (members of one batched launch whose
+  // operand views differ) share it instead of adding up.
+  constexpr int TILES = KW * 2 * (Tiles::A + Tiles::B);
+  float* const pool = lds_pool<TILES + (KW > 1 ? (KW - 1) * THREADS * TM * TN * 4 : 0)>();
+
+  // zid: the workgroup's z index within this launch (blockIdx.z, or its part
+  // below the member index in a batched launch); (tx, ty): its output tile's column
+  // and row (blockIdx.x and .y, or their XCD-grouped places).
+  const uint32_t kz = SPLIT ? zid % chunks : 0u;
+  const uint32_t bz = SPLIT ? zid / chunks : zid;
+  const uint32_t kbeg0 = SPLIT ? kz * chunkK : 0u;
+  const uint32_t kend0 = SPLIT ? min(K, kbeg0 + chunkK) : K;
+  // K groups (KW > 1, for few-tile products: more wavefronts in flight per CU): group g
+  // sums K range [kbeg0 + g·sub, kbeg0 + (g+1)·sub) of this workgroup's range, every
+  // group the same number of slices (a short last range is zero-filled, so every
+  // barrier is reached by all), and the groups' sums are added in order g = 0, 1, ...
+  // after the loop. The split depends on (M, N, K, KW) alone, as everything else here.
+  const int kg = KW == 1 ? 0 : static_cast<int>(threadIdx.x) / THREADS;
+  const uint32_t sub = KW == 1 ? kend0 - kbeg0 : ((kend0 - kbeg0 + KW * BK - 1) / (KW * BK)) * BK;
+  const uint32_t kbeg = kbeg0 + kg * sub;
+  const uint32_t kend = min(kend0, kbeg + sub);
+  const uint32_t m0 = ty * BM, n0 = tx * BN;
+  const float* __restrict__ Ab = a_ptr + AV::batch(bz);
+  const float* __restrict__ Bb = b_ptr + BV::batch(bz);
+
+  const uint32_t slices = KW == 1 ? (kend - kbeg + BK - 1) / BK : sub / BK;
+
+  const int tid = KW == 1 ? static_cast<int>(threadIdx.x) : static_cast<int>(threadIdx.x) % THREADS;
+  f4 acc[TM][TN];
+  gemm_f32_sum<TM, TN, BK, PF, AMODE, BMODE, AV, BV, WN, PRIO>(pool + kg * 2 * Tiles::A, pool + KW * 2 * Tiles::A + kg * 2 * Tiles::B, Ab,
+                                                               Bb, M, N, kbeg, kend, slices, m0, n0, tid, acc);
 
   if constexpr (KW > 1) {
     // Groups 1 .. KW-1 hand their sums to group 0 through LDS, which adds them in
@@ -440,51 +517,11 @@ __device__ __forceinline__ void gemm_f32(const Args& A, const float* __restrict_
         for (int j = 0; j < TN; ++j) acc[i][j] += red[g - 1][tid][i * TN + j];
   }
 
-  // Store: lane (t16, q) of tile (i, j) holds row t16, columns 4q .. 4q+3.
-  constexpr bool VOUT = true;
-  if (SPLIT) {
-    float* __restrict__ part = A.ws + (size_t)(kz * batch + bz) * M * N;
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const uint32_t row = m0 + wm * TM * 16 + i * 16 + t16;
-        const uint32_t col0 = n0 + wn * TN * 16 + j * 16 + 4 * q;
-        if (row >= M) continue;
-        if (N % 4 == 0 && VOUT) {
-          if (col0 < N) *reinterpret_cast<f4*>(part + (size_t)row * N + col0) = acc[i][j];
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (col0 + r < N) part[(size_t)row * N + col0 + r] = acc[i][j][r];
-        }
-      }
-    return;
-  }
-  // Epilogue: the fused body on each accumulator element, then the store.
-  const Epi epi;
-#pragma unroll
-  for (int i = 0; i < TM; ++i) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const uint32_t row = m0 + wm * TM * 16 + i * 16 + t16;
-      const uint32_t col0 = n0 + wn * TN * 16 + j * 16 + 4 * q;
-      if (row >= M) continue;
-      const uint32_t o = (bz * M + row) * N + col0;
-      if (N % 4 == 0 && VOUT) {
-        if (col0 < N) {
-          f4 v;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = epi(A, o + r, acc[i][j][r]);
-          *reinterpret_cast<f4*>(A.out + o) = v;
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (col0 + r < N) A.out[o + r] = epi(A, o + r, acc[i][j][r]);
-      }
-    }
-  }
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int wm = wave / WN, wn = wave % WN;
+  const int t16 = lane & 15, q = lane >> 4;
+  gemm_store<TM, TN, SPLIT, Epi>(A, acc, batch, M, N, kz, bz, m0 + wm * TM * 16 + t16, n0 + wn * TN * 16 + 4 * q);
 }
 
 // Output element j of a split-K matmul's product: its chunks' partial sums from the

@@ -318,11 +318,12 @@ function scratchLowerings(shapes) {
 
 /** The load modes (A, B) of a matmul launch's kernel, or null. */
 function gemmModes(l) {
-  // gemm_f32<TM, TN, BK, PF, AMODE, BMODE, SPLIT, ...>
-  const m = l.kernels[0].source.match(/gemm_f32<([^>]*)>/);
+  // gemm_f32<TM, TN, BK, PF, AMODE, BMODE, SPLIT, ...>, gemm_bf16x3<WM, WN, TM, TN, AKC, BKC, KT, AMODE, BMODE, SPLIT, ...>
+  const m = l.kernels[0].source.match(/gemm_(f32|bf16x3)<([^>]*)>/);
   if (!m) return null;
-  const a = m[1].split(',').map((x) => x.trim());
-  return [Number(a[4]), Number(a[5])];
+  const a = m[2].split(',').map((x) => x.trim());
+  const at = m[1] === 'f32' ? 4 : 7;
+  return [Number(a[at]), Number(a[at + 1])];
 }
 
 /** The K split (chunks, chunk length) of a matmul launch's kernel, or null. */

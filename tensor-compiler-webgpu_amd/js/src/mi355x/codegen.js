@@ -814,13 +814,56 @@ function gemmTiling(batch, M, N, K, tuning, peers) {
   // Unpadded products (above) take two groups up to 1024 tiles (the logits: 7.2 -> 6.7 us).
   const kw = t.kw || (T === 1 && chunks === 1 && blocks(1) <= 512 && K >= 256 ? (K >= 512 ? 4 : 2)
     : unpad && chunks === 1 && blocks(1) <= 1024 && K >= 256 ? 2 : 1);
+  const bf3 = t.bf3 === undefined && !t.tile && !t.waves && !t.kw && t.splitk === undefined && kw === 1 ? bf16x3Tiling(batch, M, N, K, P, chunks) : null;
+  if (bf3) return bf3;
   const bk = t.bk || (kw > 1 ? 32 : wn === 4 ? 32 : T === 1 ? 64 : T === 2 ? 32 : 16);
   const pf = t.pf || 2;
   const prio = t.prio !== undefined ? !!t.prio : true;
   // Per-wavefront accumulator tiles along M (tm) and N (tn): T x T unless tuned.
   const tm = t.tm || T, tn = t.tn || T;
   const wide = batch * Math.ceil(M / (32 * tm)) * Math.ceil(N / (16 * wn * tn));
-  return { T, tm, tn, chunks, chunkK, bk, pf, wn, prio, kw, blocks: wide * chunks };
+  return { T, tm, tn, chunks, chunkK, bk, pf, wn, prio, kw, bf3: !!t.bf3, blocks: wide * chunks };
+}
+
+// The tiles of tcmi_gemm_bf16x3.h's kernel, and the relative time of one on a CU per output
+// element and k, measured where each fills the chip: 8192 x 256 x 1024 (M x K x N) 30.7, 35.7
+// and 39.1 us, 8192 x 1024 x 256 (128 wide tiles: half the chip) 58, 34.8 and 38.7 us.
+const BF16X3_TILES = [{ tm: 4, tn: 4, wn: 4, cost: 1 }, { tm: 2, tn: 2, wn: 4, cost: 1.17 }, { tm: 2, tn: 2, wn: 2, cost: 1.3 }];
+
+/**
+ * The tiling of a product on the bf16 matrix cores (tcmi_gemm_bf16x3.h), or null where the
+ * fp32 kernel is the better one. Measured, fp32 against bf16 parts:
+ *   4096^3 1040 against 620 us; 8192 x 256 x 1024 43 / 30.7; 8192 x 1024 x 256 43.4 / 34.8;
+ *   8192 x 256 x 256 14.3 / 12.2; 1024^3 42.4 / 24.1; 1000 x 515 x 777 30 / 16.6;
+ *   4 weight gradients 256 x 8192 x 1024 179 / 110, 16 of 256 x 8192 x 256 165 / 119.
+ * fp32 keeps
+ *   - products it sums in K groups (few tiles): 512^3 5.2 against 12.7 us, 640^3 12.2 / 17.3;
+ *     K groups also leave it the smaller error (512^3 without its bias: 2.1e-7 against 3.4e-7);
+ *   - a K below 96 (8192 x 96 x 256 8.8 / 7.9, 1024 x 64 x 1024 5.6 / 5.6), or below 512
+ *     where the tiles do not fill the chip (768 x 256 x 768 7.9 / 9.1);
+ *   - products that would pad by more than a fifth (8192 x 256 x 96 7.9 / 8.7).
+ * Each CU runs its tiles one after another (the chip's 256 at a time), so the tile is the one
+ * with the least rounds x area x cost. K is split no less than the fp32 kernel splits it (`chunks`:
+ * the sums of shorter chunks are the more exact) and until the tiles of the products sharing
+ * the dispatch fill the chip.
+ */
+function bf16x3Tiling(batch, M, N, K, peers, chunks) {
+  if (K < 96 || Math.max(batch * M * K, batch * K * N) >= 2 ** 28) return null;
+  let best = null;
+  for (const c of BF16X3_TILES) {
+    const bm = 32 * c.tm, bn = 16 * c.wn * c.tn;
+    const rows = Math.ceil(M / bm), cols = Math.ceil(N / bn), tiles = batch * rows * cols;
+    if (rows * bm * cols * bn * 5 > 6 * M * N) continue;
+    let parts = chunks === 1 ? 1 : Math.max(chunks, Math.min(Math.ceil(256 / (tiles * peers)), Math.floor(K / 256), 32));
+    const chunkK = Math.ceil(Math.ceil(K / parts) / 32) * 32;
+    parts = Math.ceil(K / chunkK);
+    const all = tiles * parts * (chunks === 1 ? 1 : peers);
+    if (all < 128 || (all < 256 && K < 512)) continue;
+    const cost = Math.ceil(all / 256) * bm * bn * c.cost * chunkK;
+    if (!best || cost < best.cost) best = { cost, tm: c.tm, tn: c.tn, wn: c.wn, chunks: parts, chunkK, blocks: tiles * parts };
+  }
+  return best && { T: best.tm, tm: best.tm, tn: best.tn, chunks: best.chunks, chunkK: best.chunkK, bk: 32, pf: 1, wn: best.wn, prio: false, kw: 1,
+    bf3: true, blocks: best.blocks };
 }
 
 /**
@@ -829,11 +872,13 @@ function gemmTiling(batch, M, N, K, tuning, peers) {
  * each K group's A and B tiles, rows padded by 4, and the K groups' hand-over area.
  */
 function gemmPoolFloats(tl, amode, bmode) {
-  const BM = 32 * tl.tm, BN = 16 * tl.wn * tl.tn, BK = tl.bk;
+  const BM = 32 * tl.tm, BN = 16 * tl.wn * tl.tn, BK = tl.bf3 ? 16 : tl.bk;
   const aK = amode === 1, bN = bmode === 1;
   const aTile = (aK ? BK : BM) * (aK ? BM + 4 : BK + 4);
   const bTile = (bN ? BN : BK) * (bN ? BK + 4 : BN + 4);
   const threads = 128 * tl.wn;
+  // tcmi_gemm_bf16x3.h: two buffers of three bf16 parts, four planes of 16 bytes a line each.
+  if (tl.bf3) return Math.max(2 * 12 * (BM + BN) * 16 / 4, 2 * (aTile + bTile));
   return tl.kw * 2 * (aTile + bTile) + (tl.kw > 1 ? (tl.kw - 1) * threads * tl.tm * tl.tn * 4 : 0);
 }
 
@@ -898,7 +943,7 @@ function operandView(name, view, batchDims, R, C) {
 };
 `;
     const span = (fs) => fs.reduce((t, [e, st]) => t + (e - 1) * st, 0);
-    return { text, mode, limit: 1 + batchLimit + span(rf) + span(cf), mapped: true };
+    return { text, mode, limit: 1 + batchLimit + span(rf) + span(cf), mapped: true, rows: mode === 1, cols: mode === 0 };
   }
   const others4 = (x) => strides.every((s) => s % 4 === 0) && x % 4 === 0;
   let mode = 2;
@@ -911,7 +956,8 @@ function operandView(name, view, batchDims, R, C) {
 `;
   // One past the largest element offset the kernel can address.
   const limit = 1 + batchLimit + (R - 1) * v.sr + (C - 1) * v.sc;
-  return { text, mode, limit };
+  // rows, cols: whether that index is the contiguous one, whatever the alignment.
+  return { text, mode, limit, rows: v.sr === 1, cols: v.sc === 1 };
 }
 
 /**
@@ -1000,13 +1046,17 @@ ${indent(lines, '    ')}
   // The tile's place passed explicitly: a ragged batch runs this text with blockIdx
   // standing for the member's own place (raggedKernel).
   const place = grouped ? ', wg.z, wg.x, wg.y' : ', blockIdx.z, blockIdx.x, blockIdx.y';
+  const call = tl.bf3
+    ? `tcmi::gemm_bf16x3<2, ${tl.wn}, ${tl.tm}, ${tl.tn}, ${av.cols}, ${bv.rows}, ${tl.chunkK % 32 !== 0 || K % 32 !== 0}, ${av.mode}, ${bv.mode}, ${split}, __KERNEL___av, __KERNEL___bv, __KERNEL___epi>(A, A.in[${ia}], A.in[${ib}],
+      ${4 * av.limit}u, ${4 * bv.limit}u, `
+    : `tcmi::gemm_f32<${tl.tm}, ${tl.tn}, ${tl.bk}, ${tl.pf}, ${av.mode}, ${bv.mode}, ${split}, __KERNEL___av, __KERNEL___bv, __KERNEL___epi${variant}>(A, A.in[${ia}], A.in[${ib}],
+      `;
   const main = `extern "C" __global__ void __launch_bounds__(${threads}) __KERNEL__(const TcmiArgs A) {
 ${grouped ? `  ${XCD_GROUPED}
-` : ''}  tcmi::gemm_f32<${tl.tm}, ${tl.tn}, ${tl.bk}, ${tl.pf}, ${av.mode}, ${bv.mode}, ${split}, __KERNEL___av, __KERNEL___bv, __KERNEL___epi${variant}>(A, A.in[${ia}], A.in[${ib}],
-      ${batch}u, ${M}u, ${K}u, ${N}u, ${tl.chunks}u, ${tl.chunkK}u${place});
+` : ''}  ${call}${batch}u, ${M}u, ${K}u, ${N}u, ${tl.chunks}u, ${tl.chunkK}u${place});
 }
 `;
-  const text = `#include "tcmi_gemm.h"\n${av.text}${bv.text}${epi}${main}`;
+  const text = `#include "${tl.bf3 ? 'tcmi_gemm_bf16x3.h' : 'tcmi_gemm.h'}"\n${av.text}${bv.text}${epi}${main}`;
   const k = kernelText('mm', text);
   const kernels = [{ name: k.name, source: k.source, grid: [Math.ceil(N / (16 * tl.wn * tl.tn)), Math.ceil(M / (32 * tl.tm)), batch * tl.chunks],
     block: [threads, 1, 1], lds: 0, pool: gemmPoolFloats(tl, av.mode, bv.mode) }];

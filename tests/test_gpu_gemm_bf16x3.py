@@ -1,0 +1,157 @@
+"""The matmul on the bf16 matrix cores (csrc/kernels/tcmi_gemm_bf16x3.h) where it can go
+wrong: tiles, slices and loads that end inside a product, both transposed forms, batches, the K
+split, operands the split into bf16 parts does not cover (infinities, NaN, values near the
+largest and the smallest float32), and its error beside the fp32 kernel's."""
+import ctypes
+import pathlib
+
+import numpy as np
+import pytest
+
+from oracle import bounds
+from test_zz_no_alloc import ARG_BYTES, pack
+
+pytestmark = pytest.mark.gpu
+
+PKG = pathlib.Path(__file__).resolve().parent.parent / "tensor-compiler-webgpu_amd"
+
+# (M, K, N): one past and one short of the 128 x 256, 64 x 128 and 64 x 64 tiles, K ending 1, 3
+# and 31 short of a slice of 32 and a group of 4, rows of odd length (unaligned 128-bit loads).
+RAGGED = [(1000, 777, 515), (1025, 513, 767), (1087, 515, 1024), (961, 545, 1026), (4095, 97, 1021)]
+
+
+def test_forward_and_both_transposed_products_within_budget(tmp_path, tool):
+    import tcmi_bridge
+    print("gpu step: gpu-configs, ragged products forward and gradient", flush=True)
+    tool("gpu-configs", {"c4": [{"act": "tanh", "M": M, "K": K, "N": N, "rows": 24, "cols": 24} for M, K, N in RAGGED],
+                         "unfused": True}, out=str(tmp_path), timeout=600)
+    b = tcmi_bridge.Bundle(tmp_path)
+    assert len(b.cases) == 2 * len(RAGGED)
+    for c in b.cases:
+        assert c["canaryFused"] and c["canaryUnfused"] and c["perf"]["canary"], c["name"]
+        assert c["perf"]["same"] == c["perf"]["total"], (c["name"], c["perf"])
+        for s in c["samples"]:
+            ins = {k: b.arr(v) for k, v in s["inputs"].items()}
+            ids = [x["id"] for x in s["compare"]]
+            ref = bounds.streaming_reference(s["graph"], ins, ids)
+            j = bounds.judge_outputs([ref[i][0] for i in ids], [ref[i][1] for i in ids], [b.arr(x["fused"]) for x in s["compare"]])
+            assert j["pass"], (c["name"], s["slice"], j["first"], j["unjudged"])
+
+
+def product(tool, x, w):
+    """x [.., M, K] times w [.., K, N] by the plain lowering's kernels, in this process; and their text."""
+    import tcmi_ctypes
+    u32, u64 = tcmi_ctypes.u32, tcmi_ctypes.u64
+    shape = list(x.shape[:-1]) + [w.shape[-1]]
+    graph = {"nodes": [{"op": "input", "inputs": [], "attrs": {"name": "x", "shape": list(x.shape)}, "shape": list(x.shape)},
+                       {"op": "input", "inputs": [], "attrs": {"name": "w", "shape": list(w.shape)}, "shape": list(w.shape)},
+                       {"op": "matmul", "inputs": [0, 1], "attrs": {}, "shape": shape}]}
+    launch = tool("lower", {"graph": graph, "sources": True})["launches"][0]
+    t = tcmi_ctypes.load()
+    t.init()
+    t.set_include_dir(str(PKG / "csrc" / "kernels").encode())
+    t.set_cache_dir(str(PKG / "_build" / "kcache").encode())
+    mod = u64()
+    text = '#include "tcmi_device.h"\n' + "\n".join(k["source"] for k in launch["kernels"])
+    t.module_compile(text.encode(), None, ctypes.byref(mod))
+    owned = []
+
+    def alloc(nbytes):
+        h = u64()
+        t.malloc((nbytes + 15) // 16 * 16, ctypes.byref(h))
+        owned.append(h.value)
+        return h.value
+
+    try:
+        y = np.empty(shape, dtype=np.float32)
+        hx, hw, hy, ws = alloc(x.nbytes), alloc(w.nbytes), alloc(y.nbytes), alloc(max(16, launch["workspace"]))
+        for h, v in ((hx, x), (hw, w)):
+            t.h2d(h, 0, np.ascontiguousarray(v).ctypes.data, v.nbytes)
+        a = pack([hx, hw], hy, ws, launch["params"])
+        for k in launch["kernels"]:
+            f = u64()
+            t.module_function(mod.value, k["name"].encode(), ctypes.byref(f))
+            t.launch(f.value, (u32 * 3)(*k["grid"]), (u32 * 3)(*k["block"]), k["lds"], a.ctypes.data, ARG_BYTES)
+        t.sync()
+        t.d2h(y.ctypes.data, hy, 0, y.nbytes)
+        return y, text
+    finally:
+        for h in owned:
+            t.free(h)
+        t.module_unload(mod)
+
+
+@pytest.mark.parametrize("batch,M,K,N", [(1, 768, 512, 768), (1, 4097, 96, 1024), (1, 256, 8192, 512), (3, 520, 530, 900), (1, 1024, 4096, 2048)])
+def test_sums_are_no_less_exact_than_fp32_ones(tool, batch, M, K, N):
+    """Every element within gamma(K) of float64's, and their 2-norm error within what an fp32 sum of K terms makes: K
+    roundings of 2^-24 / sqrt(3) of the partial sum, whose square grows as k / K (K / 2 in all), and the result's own."""
+    print(f"gpu step: product {batch}x{M}x{K}x{N}", flush=True)
+    rng = np.random.default_rng(M + K + N)
+    lead = (batch,) if batch > 1 else ()
+    x = rng.standard_normal(lead + (M, K)).astype(np.float32)
+    w = rng.standard_normal(lead + (K, N)).astype(np.float32)
+    y, text = product(tool, x, w)
+    assert "gemm_bf16x3" in text
+    exact = x.astype(np.float64) @ w.astype(np.float64)
+    u = 2.0 ** -24
+    assert np.all(np.abs(y - exact) <= K * u / (1 - K * u) * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64)))
+    rel = np.linalg.norm(y - exact) / np.linalg.norm(exact)
+    assert rel <= u * np.sqrt(K / 2 / 3 + 1), rel
+
+
+def test_selection_returns_the_values_bit_for_bit(tool):
+    """A product with the identity's first columns: the three parts sum back to the value. Values over
+    60 binades, zeros of both signs."""
+    print("gpu step: selection 1024x544x640", flush=True)
+    rng = np.random.default_rng(5)
+    x = (rng.standard_normal((1024, 544)) * 2.0 ** rng.integers(-30, 30, (1024, 544))).astype(np.float32)
+    x[::7, ::5] = 0.0
+    y, text = product(tool, x, np.eye(544, 640, dtype=np.float32))
+    assert "gemm_bf16x3" in text
+    want = np.zeros((1024, 640), dtype=np.float32)
+    want[:, :544] = x
+    assert np.array_equal(y, want)
+
+
+@pytest.mark.parametrize("what", ["infinite", "nan", "near the largest", "overflowing", "tiny", "subnormal results", "wide"])
+def test_values_the_parts_do_not_cover_take_the_fp32_sums(tool, what):
+    """One such row (and one column) among ordinary ones: IEEE results where they are not finite, fp32's accuracy
+    where they are."""
+    print(f"gpu step: 1024x512x640, {what}", flush=True)
+    rng = np.random.default_rng(9)
+    x = rng.standard_normal((1024, 512)).astype(np.float32)
+    w = rng.standard_normal((512, 640)).astype(np.float32)
+    if what == "infinite":
+        x[130, 7], w[9, 300] = np.inf, -np.inf
+    elif what == "nan":
+        x[130, 7] = np.nan
+    elif what == "near the largest":
+        x[130, :] = 0.0
+        x[130, 7] = np.float32(3.4028235e38)      # rounds to infinity in bf16
+        w[7, :] = np.where(np.abs(w[7, :]) < 0.9, w[7, :], 0.5)
+    elif what == "overflowing":
+        x[130, 7], w[7, :] = 1e30, 1e30
+    elif what == "tiny":
+        x[130, :] = (rng.standard_normal(512) * 1e-35).astype(np.float32)
+        x[500, :] = (rng.standard_normal(512) * 1e-32).astype(np.float32)
+    elif what == "subnormal results":
+        x[130, :] = (rng.standard_normal(512) * 1e-38).astype(np.float32)
+    elif what == "wide":
+        x[130, :] = (rng.standard_normal(512) * 1e-34).astype(np.float32)
+        w[:, 300] = (rng.standard_normal(512) * 1e34).astype(np.float32)
+    y, text = product(tool, x, w)
+    assert "gemm_bf16x3" in text
+    with np.errstate(invalid="ignore", over="ignore"):
+        exact = x.astype(np.float64) @ w.astype(np.float64)
+        want = exact.astype(np.float32)
+    finite = np.isfinite(want)
+    assert np.array_equal(np.isnan(y), np.isnan(want))
+    assert np.array_equal(y[~finite & ~np.isnan(want)], want[~finite & ~np.isnan(want)])
+    # Finite sums: 512 fp32 roundings of each product and partial sum; a subnormal may be flushed to 0.
+    budget = 512 * 2.0 ** -24 * (np.abs(np.nan_to_num(x, posinf=0, neginf=0)).astype(np.float64)
+                                 @ np.abs(np.nan_to_num(w, posinf=0, neginf=0)).astype(np.float64)) + 2.0 ** -126
+    assert np.all(np.abs(y[finite] - exact[finite]) <= budget[finite])
+    if what in ("tiny", "wide"):   # 1e-35 has no third part in bf16; fp32 keeps all its bits
+        # (a row of 1e-32 keeps them too): 2-norm errors as an ordinary row's
+        for r in (130, 500) if what == "tiny" else (130,):
+            assert np.linalg.norm(y[r] - exact[r]) <= 1e-6 * np.linalg.norm(exact[r]), r
