@@ -1416,13 +1416,14 @@ async function main() {
       break;
     }
     case 'batch-check': {
-      // Batched launches of model steps and corpus programs (perf lowering), checked against
-      // the plain order; with `plant`, the planted mistakes of batch_check.js as well.
+      // Batched launches of model steps, corpus programs and given graphs ({ name, graph, keep };
+      // perf lowering), checked against the plain order; with `plant`, the planted mistakes of batch_check.js as well.
       const { checkBatches, plantBatchMistake } = require('../src/testing/batch_check');
       const one = (name, graph, keep) => {
         const plain = lowerMI355X(graph, { perf: true, keep, batch: false, absorb: true });
         const batched = lowerMI355X(graph, { perf: true, keep, absorb: true });
-        const res = { name, launches: batched.launches.length, check: checkBatches(plain, batched) };
+        const res = { name, launches: batched.launches.length, check: checkBatches(plain, batched),
+          merged: (batched.batches || []).filter((b) => b.merged).map((b) => ({ count: b.count, kind: batched.launches[b.start].kind, kernel: b.kernels[0].name })) };
         if (req.plant) {
           for (const kind of ['dependent', 'early', 'grid', 'body']) {
             const bad = plantBatchMistake(batched, kind);
@@ -1446,6 +1447,10 @@ async function main() {
             out.push(one(`corpus-${i}-${c.label}`, f.graph, c.keep.map((id) => f.index.get(id))));
           }
         }
+      }
+      for (const c of req.graphs || []) {
+        const f = fuse(Graph.fromJSON(c.graph), { keep: c.keep });
+        out.push(one(c.name, f.graph, c.keep.map((id) => f.index.get(id))));
       }
       break;
     }

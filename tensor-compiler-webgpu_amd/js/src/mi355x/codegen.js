@@ -245,6 +245,22 @@ const indent = (lines, pad) => lines.map((l) => pad + l).join('\n');
  */
 function elementwiseKernel(b, output, outShape, opts) {
   const o = opts || {};
+  // Non-temporal stores unless the lowering says the next launch reads the output
+  // (streamOut false), which then finds it in the caches; tuning nt forces either way.
+  const nt = (o.tuning || {}).nt === undefined ? o.streamOut !== false : !!o.tuning.nt;
+  checkOperands(b);
+  const k = elementwiseText(b, [{ id: output, ptr: 'A.out', nt }], outShape, o, { args: 'TcmiArgs A', kind: 'ew', at: (q) => `A.in[${q}]` });
+  // What a merged batch (mergedKernel) forms this launch again from.
+  k.merge = { body: b, output, shape: outShape, tuning: o.tuning, streamed: o.lastReads || [], nt, sabotage: o.sabotage };
+  return k;
+}
+
+/**
+ * The elementwise kernel storing each of `outs` ({ id: its node, ptr: its buffer, nt: stored
+ * non-temporally }), all of outShape; `form`: the kernel's argument (args), its name's kind, and
+ * the pointer expression of operand q (at).
+ */
+function elementwiseText(b, outs, outShape, o, form) {
   const tune = o.tuning || {};
   const n = size(outShape);
   const large = n >= 2 ** 25;
@@ -252,15 +268,11 @@ function elementwiseKernel(b, output, outShape, opts) {
   // three-operand kernel at 8192 blocks (one group a thread taken, the second guarded out:
   // the difference is the compiled loop), neutral on the small kernels of the training steps.
   const U = tune.unroll || 2;
-  // Non-temporal stores unless the lowering says the next launch reads the output
-  // (streamOut false), which then finds it in the caches; tuning nt forces either way.
-  const nt = tune.nt === undefined ? o.streamOut !== false : !!tune.nt;
   // Non-temporal loads: every full-size operand (tuning ntl), or those at the positions
   // `o.lastReads` lists (the lowering's last reads of their buffers).
   const ntlAt = new Set(tune.ntl ? [] : (o.lastReads || []));
   const ntl = (k) => !!tune.ntl || ntlAt.has(k);
   const maxBlocks = tune.blocks || (large ? 512 : 8192);
-  checkOperands(b);
   if (n >= 2 ** 31) throw new Error(`elementwise kernel over ${n} elements exceeds the 32-bit index space`);
   const params = [n];
 
@@ -280,28 +292,28 @@ function elementwiseKernel(b, output, outShape, opts) {
   const vecEmitter = new Emitter(b, params, {
     load(k, ctx, lines) {
       if (ctx.root) {
-        const load = ntl(k) ? `__builtin_nontemporal_load(reinterpret_cast<const tcmi::f4*>(A.in[${k}]) + v)`
-          : `reinterpret_cast<const tcmi::f4*>(A.in[${k}])[v]`;
+        const load = ntl(k) ? `__builtin_nontemporal_load(reinterpret_cast<const tcmi::f4*>(${form.at(k)}) + v)`
+          : `reinterpret_cast<const tcmi::f4*>(${form.at(k)})[v]`;
         return `${hoistAs(`full${k}`, 'tcmi::f4', load)}[j][l]`;
       }
       const g = ctx.gather;
       if (ctx.parent && ctx.parent.root && g) {
-        if (g.g.mode === 'zero') return `${hoistAs(`zero${k}`, 'float', `A.in[${k}][0]`)}[j]`;
+        if (g.g.mode === 'zero') return `${hoistAs(`zero${k}`, 'float', `${form.at(k)}[0]`)}[j]`;
         if (g.g.mode === 'span' && g.g.inner === 1 && g.g.extent % 4 === 0) {
           return `${hoistAs(`spanv${k}|${ctx.key}`, 'tcmi::f4',
-            `reinterpret_cast<const tcmi::f4*>(A.in[${k}])[(i0 % ${g.g.extent}u) >> 2]`)}[j][l]`;
+            `reinterpret_cast<const tcmi::f4*>(${form.at(k)})[(i0 % ${g.g.extent}u) >> 2]`)}[j][l]`;
         }
         if (g.g.mode === 'span' && g.g.inner % 4 === 0) {
-          return `${hoistAs(`spans${k}|${ctx.key}`, 'float', `A.in[${k}][(i0 / ${g.g.inner}u) % ${g.g.extent}u]`)}[j]`;
+          return `${hoistAs(`spans${k}|${ctx.key}`, 'float', `${form.at(k)}[(i0 / ${g.g.inner}u) % ${g.g.extent}u]`)}[j]`;
         }
       }
       const v = `L${lines.length}_${k}`;
-      lines.push(`const float ${v} = A.in[${k}][${ctx.idx}];`);
+      lines.push(`const float ${v} = ${form.at(k)}[${ctx.idx}];`);
       return v;
     },
   });
   const lane = [];
-  const vout = vecEmitter.value(output, { key: 'i', idx: 'i', root: true, limit: n }, lane);
+  const vouts = outs.map((x) => vecEmitter.value(x.id, { key: 'i', idx: 'i', root: true, limit: n }, lane));
 
   // Scalar tail: the same body, every load scalar. The reference's sabotage
   // 'fused-bounds-off-by-one' (codegen-fused.js:160) lets one thread past the
@@ -313,18 +325,24 @@ function elementwiseKernel(b, output, outShape, opts) {
   const tailEmitter = new Emitter(b, params, {
     load(k, ctx, lines) {
       const v = `T${lines.length}_${k}`;
-      lines.push(`const float ${v} = A.in[${k}][${ctx.idx}];`);
+      lines.push(`const float ${v} = ${form.at(k)}[${ctx.idx}];`);
       return v;
     },
   }, offByOne ? 1 : 0);
   tailEmitter.gatherBase = vecEmitter.gatherBase;  // same parameter offsets
   const tail = [];
-  const tout = tailEmitter.value(output, { key: 'i', idx: 'i', root: true, limit: offByOne ? n + 1 : n }, tail);
+  const touts = outs.map((x) => tailEmitter.value(x.id, { key: 'i', idx: 'i', root: true, limit: offByOne ? n + 1 : n }, tail));
 
   const guard = offByOne ? 'threadIdx.x <= (n & 3u)' : 'threadIdx.x < (n & 3u)';
-  const store = nt ? '__builtin_nontemporal_store(o4, reinterpret_cast<tcmi::f4*>(A.out) + v);'
-    : 'reinterpret_cast<tcmi::f4*>(A.out)[v] = o4;';
-  const text = `extern "C" __global__ void __launch_bounds__(${WG}) __KERNEL__(const TcmiArgs A) {
+  // The outputs' registers: r (o4) for a single one.
+  const q = (x) => (outs.length === 1 ? '' : `${x}_`);
+  const stores = [];
+  outs.forEach((x, i) => {
+    const o4 = `${outs.length === 1 ? 'o4' : `o4_${i}`}`, r = outs.length === 1 ? 'r' : `r${q(i)}`;
+    stores.push(`const tcmi::f4 ${o4} = {${r}[0], ${r}[1], ${r}[2], ${r}[3]};`,
+      x.nt ? `__builtin_nontemporal_store(${o4}, reinterpret_cast<tcmi::f4*>(${x.ptr}) + v);` : `reinterpret_cast<tcmi::f4*>(${x.ptr})[v] = ${o4};`);
+  });
+  const text = `extern "C" __global__ void __launch_bounds__(${WG}) __KERNEL__(const ${form.args}) {
   const uint32_t n = ${n}u;
   const uint32_t nv = n >> 2;
   const uint32_t stride = gridDim.x * ${WG}u;
@@ -343,26 +361,25 @@ ${indent(hoist, '        ')}
       const uint32_t v = base + j * stride;
       if (v < nv) {
         const uint32_t i0 = v << 2;
-        float r[4];
+        float ${outs.map((x, i) => `r${q(i)}[4]`).join(', ')};
 #pragma unroll
         for (int l = 0; l < 4; ++l) {
           const uint32_t i = i0 + l;
 ${indent(lane, '          ')}
-          r[l] = ${vout};
+${outs.map((x, i) => `          r${q(i)}[l] = ${vouts[i]};`).join('\n')}
         }
-        const tcmi::f4 o4 = {r[0], r[1], r[2], r[3]};
-        ${store}
+${indent(stores, '        ')}
       }
     }
   }
   if (blockIdx.x == 0 && ${guard}) {
     const uint32_t i = (nv << 2) + threadIdx.x;
 ${indent(tail, '    ')}
-    A.out[i] = ${tout};
+${outs.map((x, i) => `    ${x.ptr}[i] = ${touts[i]};`).join('\n')}
   }
 }
 `;
-  const k = kernelText('ew', text);
+  const k = kernelText(form.kind, text);
   const groups = Math.max(1, Math.min(Math.ceil(Math.max(1, n >> 2) / WG), maxBlocks));
   return { name: k.name, source: k.source, params: Uint32Array.from(params), grid: [groups, 1, 1], block: [WG, 1, 1], lds: 0, workspace: 0,
     needsPad: offByOne };
@@ -386,14 +403,20 @@ const isReduce = (n) => n.op === 'sum' || n.op === 'max';
  */
 function rowwiseKernel(b, output, opts) {
   const o = opts || {};
+  checkOperands(b);
+  // Full-size output that the next launch does not read: stored non-temporally, so it
+  // does not displace data that launch reads from the caches (tuning nto forces either way).
+  const nt = (o.tuning || {}).nto === undefined ? o.streamOut === true : !!o.tuning.nto;
+  const k = rowwiseText(b, [{ id: output, ptr: 'A.out', nt }], o, { args: 'TcmiArgs A', kind: 'row', at: (q) => `A.in[${q}]` });
+  k.merge = { body: b, output, rows: k.rows, held: k.held, tuning: o.tuning, streamed: o.lastReads || [], nt, sabotage: o.sabotage };
+  return k;
+}
+
+/** The rowwise kernel storing each of `outs`, as elementwiseText's outs and form. */
+function rowwiseText(b, outs, o, form) {
   // Operand positions whose full-size loads are the lowering's last reads of their
   // buffers: loaded non-temporally (row length a multiple of 4 only).
   const streamed = new Set(o.lastReads || []);
-  // Full-size output that the next launch does not read: stored non-temporally, so it
-  // does not displace data that launch reads from the caches (tuning nto forces either way).
-  const tuneRow = o.tuning || {};
-  const ntOut = tuneRow.nto === undefined ? o.streamOut === true : !!tuneRow.nto;
-  checkOperands(b);
   const reductions = b.nodes.filter(isReduce);
   if (!reductions.length) throw new Error('rowwise kernel without a reduction');
   const S = b.nodes[reductions[0].inputs[0]].shape;
@@ -413,7 +436,7 @@ function rowwiseKernel(b, output, opts) {
   const E = Math.max(1, Math.ceil(C / (W * T)));  // slots per thread
   const params = [R, C];
   const rowTier = (id) => size(b.nodes[id].shape) === R && size(b.nodes[id].shape) !== R * C;
-  const outRow = rowTier(output) || (R === size(b.nodes[output].shape) && C !== 1 && size(b.nodes[output].shape) !== R * C);
+  const outRow = (id) => rowTier(id) || (R === size(b.nodes[id].shape) && C !== 1 && size(b.nodes[id].shape) !== R * C);
 
   // Loads at the element index: cached per load site in registers. `fills` keeps
   // each cache's kind in first-use order; the kernel text declares and fills them.
@@ -452,7 +475,7 @@ function rowwiseKernel(b, output, opts) {
         let v = `R${rowLines.length}_${k}`;
         if (rowNames.has(v)) v = `${v}_${rowNames.size}`;
         rowNames.add(v);
-        lines.push(`const float ${v} = A.in[${k}][${ctx.idx}];`);
+        lines.push(`const float ${v} = ${form.at(k)}[${ctx.idx}];`);
         return v;
       }
       if (ctx.root) {
@@ -466,7 +489,7 @@ function rowwiseKernel(b, output, opts) {
         return `tcmi::lane4(${cache(`col${k}`, k, 'col')}[s], l)`;
       }
       const v = `L${lines.length}_${k}`;
-      lines.push(`const float ${v} = A.in[${k}][${ctx.idx}];`);
+      lines.push(`const float ${v} = ${form.at(k)}[${ctx.idx}];`);
       return v;
     },
   };
@@ -476,16 +499,16 @@ function rowwiseKernel(b, output, opts) {
     if (f.mode === 'nt') {
       return head.concat([`for (int s = 0; s < ${E}; ++s) { const uint32_t c0 = (ln + s * ${T}u) * 4u;`,
         `  tcmi::f4 t = {0.f, 0.f, 0.f, 0.f};`,
-        `  if (c0 < C) t = __builtin_nontemporal_load(reinterpret_cast<const tcmi::f4*>(A.in[${f.k}] + rowBase) + (c0 >> 2));`,
+        `  if (c0 < C) t = __builtin_nontemporal_load(reinterpret_cast<const tcmi::f4*>(${form.at(f.k)} + rowBase) + (c0 >> 2));`,
         `  ${dst}[s] = make_float4(t[0], t[1], t[2], t[3]); }`]);
     }
     if (f.mode === 'vec' || f.mode === 'col') {
-      const src = f.mode === 'col' ? `A.in[${f.k}]` : `A.in[${f.k}] + rowBase`;
+      const src = f.mode === 'col' ? `${form.at(f.k)}` : `${form.at(f.k)} + rowBase`;
       return head.concat([`for (int s = 0; s < ${E}; ++s) { const uint32_t c0 = (ln + s * ${T}u) * 4u;`,
         `  ${dst}[s] = c0 < C ? reinterpret_cast<const float4*>(${src})[c0 >> 2] : make_float4(0.f, 0.f, 0.f, 0.f); }`]);
     }
     return head.concat([`for (int s = 0; s < ${E}; ++s) { const uint32_t c0 = ln + s * ${T}u;`,
-      `  ${dst}[s] = c0 < C ? A.in[${f.k}][rowBase + c0] : 0.f; }`]);
+      `  ${dst}[s] = c0 < C ? ${form.at(f.k)}[rowBase + c0] : 0.f; }`]);
   };
   const cacheType = (f) => (f.mode === 'scalar' ? 'float' : 'float4');
   em = new Emitter(b, params, hooks);
@@ -532,21 +555,22 @@ ${indent(bodyLines, '    ')}
       `const float red${k} = ${result};`);
     reduced.set(rd.id, `red${k}`);
   });
-  for (const key of Array.from(em.memo.keys())) if (key.startsWith('e')) em.memo.delete(key);
-  let store;
-  if (outRow) {
+  const store = [];
+  for (const out of outs) {
+    for (const key of Array.from(em.memo.keys())) if (key.startsWith('e')) em.memo.delete(key);
     const rowBefore = rowLines.length;
-    const v = em.value(output, ROW, rowLines);
-    const pre = rowLines.splice(rowBefore);
-    store = [...pre, `if (ln == 0) A.out[r] = ${v};`];
-  } else {
-    const rowBefore = rowLines.length;
+    if (outRow(out.id)) {
+      const v = em.value(out.id, ROW, rowLines);
+      const pre = rowLines.splice(rowBefore);
+      store.push(...pre, `if (ln == 0) ${out.ptr}[r] = ${v};`);
+      continue;
+    }
     const inner = [];
-    const v = em.value(output, elemCtx(), inner);
+    const v = em.value(out.id, elemCtx(), inner);
     const pre = rowLines.splice(rowBefore);
     if (vec) {
       // Compute the 4 lanes of each slot, then one 128-bit store.
-      store = [...pre, `#pragma unroll
+      store.push(...pre, `#pragma unroll
 for (int s = 0; s < ${E}; ++s) {
   const uint32_t c0 = (ln + s * ${T}u) * 4u;
   if (c0 < C) {
@@ -558,17 +582,17 @@ for (int s = 0; s < ${E}; ++s) {
 ${indent(inner, '      ')}
       o4[l] = ${v};
     }
-    ${ntOut ? '__builtin_nontemporal_store(tcmi::f4{o4[0], o4[1], o4[2], o4[3]}, reinterpret_cast<tcmi::f4*>(A.out + rowBase) + (c0 >> 2));'
-    : 'reinterpret_cast<float4*>(A.out + rowBase)[c0 >> 2] = make_float4(o4[0], o4[1], o4[2], o4[3]);'}
+    ${out.nt ? `__builtin_nontemporal_store(tcmi::f4{o4[0], o4[1], o4[2], o4[3]}, reinterpret_cast<tcmi::f4*>(${out.ptr} + rowBase) + (c0 >> 2));`
+    : `reinterpret_cast<float4*>(${out.ptr} + rowBase)[c0 >> 2] = make_float4(o4[0], o4[1], o4[2], o4[3]);`}
   }
-}`];
+}`);
     } else {
-      store = [...pre, loop(inner.concat([`A.out[e] = ${v};`]))];
+      store.push(...pre, loop(inner.concat([`${out.ptr}[e] = ${v};`])));
     }
   }
   const cacheDecl = [];
   for (const f of fills) cacheDecl.push(`${cacheType(f)} ${f.c}[${E}];`, ...fillLines(f, f.c));
-  const text = `extern "C" __global__ void __launch_bounds__(${BLOCK}) __KERNEL__(const TcmiArgs A) {
+  const text = `extern "C" __global__ void __launch_bounds__(${BLOCK}) __KERNEL__(const ${form.args}) {
 ${T === 256 ? '  __shared__ float red[4];\n' : ''}  const uint32_t R = ${R}u;
   const uint32_t C = ${C}u;
   const uint32_t ln = threadIdx.x % ${T}u;     // lane within the row's group
@@ -580,10 +604,11 @@ ${indent(store, '    ')}
   }
 }
 `;
-  const k = kernelText('row', text);
+  const k = kernelText(form.kind, text);
   const cap = (o.tuning && o.tuning.blocks) || 65536;
   const groups = Math.max(1, Math.min(Math.ceil(R / G), cap));
-  return { name: k.name, source: k.source, params: Uint32Array.from(params), grid: [groups, 1, 1], block: [BLOCK, 1, 1], lds: 0, workspace: 0 };
+  return { name: k.name, source: k.source, params: Uint32Array.from(params), grid: [groups, 1, 1], block: [BLOCK, 1, 1], lds: 0, workspace: 0,
+    rows: [R, C], held: fills.length * E * W };
 }
 
 // ---- column reductions (sum / max over a non-last axis) --------------------------------
@@ -1576,6 +1601,9 @@ function batchable(k, count) {
 /** The statement that opens a kernel whose workgroups take XCD-grouped places. */
 const XCD_GROUPED = 'const tcmi::Wg wg = tcmi::xcd_grouped();';
 
+/** Whether kernel `k` may only run in a batch that computes its members together (mergedKernel). */
+function mergeOnly(k) { return /^tcmi_row_[0-9a-f]+$/.test(k.name) && !!k.merge && /__shared__/.test(k.source); }
+
 /**
  * The family of kernel `k` for batching: its text with its operand view structs taken out
  * and its own name blanked. Launches of one family differ at most in how their matmul
@@ -1591,6 +1619,9 @@ function batchFamily(k) {
   if (/^tcmi_row_[0-9a-f]+$/.test(k.name) && !k.lds && !k.ldsStatic && !/__shared__/.test(k.source)) {
     return `row@${k.grid.join(',')}/${k.block.join(',')}`;
   }
+  // Rowwise kernels that reduce a row across a workgroup fill the chip each: they are grouped
+  // only to be computed together (mergedKernel).
+  if (mergeOnly(k)) return `rows@${k.grid.join(',')}/${k.block.join(',')}`;
   // Matmul tiles take their LDS from a pool shared by instantiations of one size
   // (tcmi::lds_pool); other kernels' views would each add their own LDS: one text a family.
   if (!/^tcmi_mm_[0-9a-f]+$/.test(k.name)) return `${k.name}@${k.grid.join(',')}/${k.block.join(',')}/${k.lds}`;
@@ -1665,6 +1696,79 @@ function batchedKernel(members, count) {
   const b = kernelText(`b${k.name.split('_')[1]}`, text);
   return { name: b.name + (suffix || ''), source: b.source, grid: [k.grid[0], k.grid[1], Z * count], block: k.block.slice(), lds: k.lds,
     members: count, variants: variants.length > 1 ? variantOf.map((v) => variants[v].name) : undefined };
+}
+
+// ---- merged batches -------------------------------------------------------------------
+
+// Workgroups a merged batch's dispatch has at least (one member's grid must fill the chip by
+// itself), its members, and the floats of operand rows a lane of a merged rowwise kernel holds in
+// registers (where no member holds more).
+const MERGED_MIN_BLOCKS = 512;
+const MERGED_MAX_MEMBERS = 8;
+const MERGED_MAX_HELD = 64;
+
+/**
+ * The kernel of a merged batch: independent one-kernel launches over one grid and the same elements
+ * (rows), all elementwise or all rowwise, whose bodies one kernel computes
+ * together, storing each member's output. Each value is formed once, by the ops of its own
+ * launch in their order (identical values of several members are one), and each operand is
+ * loaded once, where members side by side along z (batchedKernel) load it once each.
+ * What bounds the members apart is HBM: measured merged against side by side, config 2's program
+ * 0 gradient (four chains, 537 MB apart, 268 MB together, their two exp and two tanh formed
+ * once) 73.5 -> 41.7 us, the logSoftmax backward over [16384, 4096] (y from x, dx from x and dy)
+ * 204 -> 173 us as one launch, LayerNorm's gradient over [8192, 256] (three rowwise members) 10.7
+ * -> 9.6 us. Run one after another in each workgroup instead, the later bodies' loads hitting
+ * the caches, the four chains took 60 us and the three rowwise members no less than side by side.
+ * `members`: { kernel (its launch's, with `merge`), reads (the buffer of each operand) }.
+ * null where they do not fit: other sizes or tunings, a sabotaged kernel, too many rows.
+ */
+function mergedKernel(members) {
+  const first = members[0].kernel, g = first.merge;
+  const family = batchFamily(first);
+  if (members.length < 2 || members.length > MERGED_MAX_MEMBERS || !/^(ew|rows?)@/.test(family) || first.grid[0] < MERGED_MIN_BLOCKS) return null;
+  const like = (m) => JSON.stringify([m.rows || size(m.shape), m.tuning || null]);
+  if (!members.every(({ kernel: k }) => k.merge && !k.merge.sabotage && batchFamily(k) === family && like(k.merge) === like(g))) return null;
+  const nodes = [], known = new Map(), places = [];
+  const streamed = new Set();
+  const add = (key, node) => {
+    if (!known.has(key)) {
+      known.set(key, nodes.length);
+      nodes.push(Object.assign({ id: nodes.length }, node));
+    }
+    return known.get(key);
+  };
+  const outs = members.map(({ kernel, reads }, m) => {
+    const { body, output, streamed: last, nt } = kernel.merge;
+    const at = new Map();
+    const need = new Set();
+    const visit = (id) => { if (!need.has(id)) { need.add(id); body.nodes[id].inputs.forEach(visit); } };
+    visit(output);
+    body.nodes.forEach((n, id) => {
+      if (!need.has(id)) return;
+      if (n.op === 'input') {
+        const k = Number(n.attrs.name.slice(1)), key = `in ${reads[k]} ${n.shape}`;
+        if (!known.has(key)) places.push(`B.m[${m}].in[${k}]`);
+        at.set(id, add(key, { op: 'input', inputs: [], attrs: { name: `a${places.length - 1}` }, shape: n.shape }));
+        if (last.includes(k)) streamed.add(Number(nodes[at.get(id)].attrs.name.slice(1)));
+        return;
+      }
+      const inputs = n.inputs.map((i) => at.get(i));
+      at.set(id, add(`${n.op} ${inputs} ${JSON.stringify(n.attrs)} ${n.shape}`, { op: n.op, inputs, attrs: n.attrs, shape: n.shape }));
+    });
+    return { id: at.get(output), ptr: `B.m[${m}].out`, nt };
+  });
+  const o = { tuning: g.tuning, lastReads: Array.from(streamed) };
+  const form = { args: `TcmiBatch<${members.length}> B`, at: (q) => places[q] };
+  let k;
+  try {
+    k = g.rows ? rowwiseText({ nodes }, outs, o, Object.assign(form, { kind: 'grow' })) : elementwiseText({ nodes }, outs, g.shape, o, Object.assign(form, { kind: 'gew' }));
+  } catch (e) {
+    if (e instanceof ParamOverflow) return null;
+    throw e;
+  }
+  if (k.held > MERGED_MAX_HELD && k.held > Math.max(...members.map((x) => x.kernel.merge.held)) || k.grid.join() !== first.grid.join()) return null;
+  return { name: k.name, source: k.source, grid: k.grid, block: k.block, lds: 0, members: members.length,
+    variants: members.some((x) => x.kernel.name !== first.name) ? members.map((x) => x.kernel.name) : undefined };
 }
 
 // ---- ragged batches -----------------------------------------------------------------
@@ -1768,4 +1872,4 @@ ${branches.join('\n')}
 module.exports = { elementwiseKernel, rowwiseKernel, colreduceKernels, gemmKernel, gemmTiling, attentionKernel, attentionGradKernel,
   gradPart, GRAD_PARTS, classifyGather, gatherStrides,
   literal, fnv, Emitter, ParamOverflow, WG, MAX_P, MAX_IN, MAX_BATCH, batchable, batchedKernel, batchFamily,
-  raggable, raggedFits, raggedKernel, textLds, RAGGED_MAX_BLOCKS, RAGGED_MAX_LDS, COLRED_ONE_PASS };
+  mergedKernel, mergeOnly, raggable, raggedFits, raggedKernel, textLds, RAGGED_MAX_BLOCKS, RAGGED_MAX_LDS, COLRED_ONE_PASS };

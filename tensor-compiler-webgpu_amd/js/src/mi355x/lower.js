@@ -71,6 +71,8 @@ function algorithmicBytes(graph, node, inputs) {
 
 function single(k) {
   const kernels = k.kernels || [{ name: k.name, source: k.source, grid: k.grid, block: k.block, lds: k.lds, needsPad: !!k.needsPad }];
+  // For the batch plan alone: not part of the record.
+  if (k.merge) Object.defineProperty(kernels[0], 'merge', { value: k.merge });
   return { kernels, params: k.params, workspace: k.workspace || 0, flops: k.flops || 0 };
 }
 
@@ -1244,7 +1246,7 @@ function lowerOnce(graph, opts, noAbsorb, noForm) {
   }
   const out = { launches, workspace, aliases: Array.from(plan.aliases.entries()), folded: Array.from(plan.folded), dead: Array.from(plan.dead) };
   if (opts.perf && opts.batch !== false) {
-    const b = batchPlan(launches, plan.aliases);
+    const b = batchPlan(launches, plan.aliases, (id) => 4 * size(graph.nodes[id].shape));
     out.launches = b.launches;
     out.batches = b.batches;
     for (const x of b.batches) out.workspace = Math.max(out.workspace, x.count * x.wsStride);
@@ -1279,7 +1281,7 @@ function lowerOnce(graph, opts, noAbsorb, noForm) {
  * [{ start, count, kernels, wsStride, ragged?, joint? }] } with each batch's members at
  * launches[start .. start + count).
  */
-function batchPlan(launches, aliases) {
+function batchPlan(launches, aliases, bytesOf) {
   const owner = (id) => (aliases.has(id) ? aliases.get(id) : id);
   const n = launches.length;
   const writer = new Map();
@@ -1401,6 +1403,17 @@ function batchPlan(launches, aliases) {
   // dispatch whose members' grids differ (codegen.js raggedKernel) and still stand alone.
   const raggedKey = (l) => (l.kernels.length === 1 && !l.workspace && cg.raggable(l.kernels[0]) ? `ragged@${l.kernels[0].block[0]}` : null);
   byWindows(raggedKey, (group, l) => cg.raggedFits(group.concat([l]).map((m) => m.kernels[0])), (members) => { members.ragged = true; }, true);
+  // Members that read the same operands are computed together, each operand loaded once (codegen.js
+  // mergedKernel), where that takes a fifth or more off the bytes the batch moves.
+  const merged = (u) => {
+    if (!bytesOf || u.ragged || u.some((l) => l.kernels.length !== 1 || l.workspace)) return null;
+    const total = (ids) => Array.from(new Set(ids)).reduce((q, id) => q + bytesOf(id), 0);
+    const reads = (l) => l.inputs.map(owner);
+    const outs = total(u.map((l) => l.node));
+    const apart = outs + u.reduce((q, l) => q + total(reads(l)), 0);
+    if (5 * (outs + total([].concat(...u.map(reads)))) > 4 * apart) return null;
+    return cg.mergedKernel(u.map((l) => ({ kernel: l.kernels[0], reads: reads(l) })));
+  };
   const order = [], batches = [];
   for (const u of units) {
     if (u.joint) {
@@ -1410,7 +1423,12 @@ function batchPlan(launches, aliases) {
       order.push(...u);
       continue;
     }
-    if (u.length > 1 && u.ragged) {
+    const one = u.length > 1 ? merged(u) : null;
+    if (one) {
+      batches.push({ start: order.length, count: u.length, kernels: [one], wsStride: 0, merged: true });
+    } else if (u.length > 1 && u[0].kernels.some(cg.mergeOnly)) {
+      // Launches that gain nothing side by side: each by itself, in this order.
+    } else if (u.length > 1 && u.ragged) {
       batches.push({ start: order.length, count: u.length, kernels: [cg.raggedKernel(u.map((m) => m.kernels[0]))], wsStride: 0, ragged: true });
     } else if (u.length > 1) {
       const l = u[0];

@@ -80,6 +80,66 @@ function runsOwnRaggedBody(bk, k, x, at) {
   return norm(body, m ? m[1] : null) === norm(own, x.name);
 }
 
+// What an elementwise or rowwise kernel's text stores to each of its output pointers, as the
+// number of a value in `table` (equal numbers: the same ops on the same values in the same
+// order, whatever the variables' names), with the kernel's sizes and loops under 'frame'.
+// `operand` names the buffer behind a pointer expression. Loads and stores past the caches
+// count as plain ones.
+function storedValues(source, operand, table) {
+  const intern = (t) => {
+    const k = t.replace(/\s+/g, '');
+    if (!table.has(k)) table.set(k, `#${table.size}`);
+    return table.get(k);
+  };
+  const env = new Map(), out = { frame: [] };
+  const value = (e) => intern(e.replace(/\b[A-Za-z_]\w*(?:\.m\[\d+\])?\.in\[\d+\]/g, operand).replace(/\b[A-Za-z_]\w*\b/g, (w) => (env.has(w) ? env.get(w) : w)));
+  const store = (ptr, v) => { (out[ptr] = out[ptr] || []).push(v); };
+  const P = '([\\w.[\\]]+)';
+  const rules = [
+    [/^(H\d+)\[j\] = __builtin_nontemporal_load\((.*) \+ v\);$/, (m) => env.set(m[1], value(`${m[2]}[v]`))],
+    [/^(H\d+)\[j\] = (.*);$/, (m) => env.set(m[1], value(m[2]))],
+    [/^if \(c0 < C\) t = __builtin_nontemporal_load\(reinterpret_cast<const tcmi::f4\*>\((.*) \+ rowBase\) \+ \(c0 >> 2\)\);$/, (m) => env.set('t', value(`row(${m[1]})`))],
+    [/^(X\d+)\[s\] = make_float4\(t\[0\], t\[1\], t\[2\], t\[3\]\); \}$/, (m) => env.set(m[1], env.get('t'))],
+    [/^(X\d+)\[s\] = c0 < C \? reinterpret_cast<const float4\*>\((.*) \+ rowBase\)\[c0 >> 2\] : .*$/, (m) => env.set(m[1], value(`row(${m[2]})`))],
+    [/^(X\d+)\[s\] = (.*) \}$/, (m) => env.set(m[1], value(m[2]))],
+    [/^(?:const )?float (\w+) = (.*);$/, (m) => env.set(m[1], value(m[2]))],
+    [/^(acc\d+) = (.*);$/, (m) => env.set(m[1], value(m[2]))],
+    [/^(r|r\d+_|o4)\[l\] = (.*);$/, (m) => env.set(m[1], value(m[2]))],
+    [/^const tcmi::f4 (\w+) = \{(\w+)\[0\].*$/, (m) => env.set(m[1], env.get(m[2]))],
+    [new RegExp(`^__builtin_nontemporal_store\\((\\w+), reinterpret_cast<tcmi::f4\\*>\\(${P}\\) \\+ v\\);$`), (m) => store(m[2], env.get(m[1]))],
+    [new RegExp(`^reinterpret_cast<tcmi::f4\\*>\\(${P}\\)\\[v\\] = (\\w+);$`), (m) => store(m[1], env.get(m[2]))],
+    [new RegExp(`^__builtin_nontemporal_store\\(tcmi::f4\\{o4.*\\}, reinterpret_cast<tcmi::f4\\*>\\(${P} \\+ rowBase\\) \\+ \\(c0 >> 2\\)\\);$`), (m) => store(m[1], env.get('o4'))],
+    [new RegExp(`^reinterpret_cast<float4\\*>\\(${P} \\+ rowBase\\)\\[c0 >> 2\\] = make_float4\\(o4.*\\);$`), (m) => store(m[1], env.get('o4'))],
+    [new RegExp(`^(if \\(ln == 0\\) )?${P}\\[([ier])\\] = (.*);$`), (m) => store(m[2], intern(`${m[1] || ''}${m[3]} ${value(m[4])}`))],
+  ];
+  for (const raw of source.split('\n')) {
+    const line = raw.trim();
+    const rule = rules.find(([re]) => re.test(line));
+    if (rule) rule[1](line.match(rule[0]));
+    else if (/^(__shared__ float red\[4\];|const uint32_t (n|nv|stride|R|C|ln|rowBase) =|for \(uint32_t (base|r) =)/.test(line)) out.frame.push(line);
+    else if (line && !/^(#pragma unroll|\}|\{|for \(int [sjl] = 0;|if \((v < nv|c < C|c0 < C)\) \{|const uint32_t (v|i0|i|c|c0|e) =|float4? X\d+\[|tcmi::f4 (H\d+\[|t = )|float H?\w*\[|float r|float o4|extern "C"|if \(blockIdx\.x == 0 && )/.test(line)) {
+      out.frame.push(`? ${line}`);   // a statement of no known form: never equal to another kernel's
+    }
+  }
+  return out;
+}
+
+// Whether merged batched kernel `bk` stores, as its member k's output, what that member's own
+// kernel stores, over the same sizes and loops.
+function formsOwnValues(bk, members) {
+  const table = new Map();
+  const all = storedValues(bk.source, (p) => {
+    const m = p.match(/^B\.m\[(\d+)\]\.in\[(\d+)\]$/);
+    return m && members[m[1]] ? `N${members[m[1]].reads[m[2]]}` : '?';
+  }, table);
+  return members.findIndex((x, k) => {
+    const own = storedValues(x.kernel.source, (p) => `N${x.reads[Number(p.match(/^A\.in\[(\d+)\]$/)[1])]}`, table);
+    const mine = all[`B.m[${k}].out`];
+    return !(mine && own['A.out'] && mine.length > 0 && mine.join() === own['A.out'].join() && own.frame.join('\n') === all.frame.join('\n')
+      && !own.frame.some((l) => l.startsWith('?')));
+  });
+}
+
 function checkBatches(plain, batched) {
   const alias = new Map(batched.aliases || []);
   const owner = (id) => (alias.has(id) ? alias.get(id) : id);
@@ -124,6 +184,18 @@ function checkBatches(plain, batched) {
         unitOf[b.start + k] = b.start;
       }
       if (b.kernels[0].grid.join() !== [at, 1, 1].join()) return { ok: false, why: `batch at ${b.start}: grid ${b.kernels[0].grid} for ${at} workgroups` };
+      continue;
+    }
+    if (b.merged) {
+      // Elementwise or rowwise launches of one grid, every member's values formed by one kernel.
+      const bk = b.kernels[0];
+      const ms = L.slice(b.start, b.start + b.count);
+      const odd = ms.findIndex((l) => b.kernels.length !== 1 || b.wsStride || l.kernels.length !== 1 || l.workspace || l.kernels[0].lds
+        || l.kernels[0].grid.join() !== bk.grid.join() || l.kernels[0].block.join() !== bk.block.join());
+      const bad = odd >= 0 ? odd : formsOwnValues(bk, ms.map((l) => ({ kernel: l.kernels[0], reads: l.inputs.map(owner) })));
+      if (bad >= 0) return { ok: false, why: `batch at ${b.start}: member ${bad} is not formed as its own kernel forms it` };
+      if (odd < 0 && bad === -1 && Object.keys(storedValues(bk.source, () => '?', new Map())).length !== b.count + 1) return { ok: false, why: `batch at ${b.start}: member outputs missing` };
+      for (let k = 0; k < b.count; k++) unitOf[b.start + k] = b.start;
       continue;
     }
     if (b.kernels.length !== first.kernels.length) return { ok: false, why: `batch at ${b.start}: ${b.kernels.length} batched kernels for ${first.kernels.length}` };
