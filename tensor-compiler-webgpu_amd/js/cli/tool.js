@@ -1416,12 +1416,12 @@ async function main() {
       break;
     }
     case 'batch-check': {
-      // Batched launches of model steps, corpus programs and given graphs ({ name, graph, keep };
-      // perf lowering), checked against the plain order; with `plant`, the planted mistakes of batch_check.js as well.
+      // Batched launches of model steps, corpus programs and given graphs ({ name, graph, keep }, lowered
+      // as the bench lowers them: nothing absorbed; perf lowering), checked against the plain order; with `plant`, the planted mistakes of batch_check.js as well.
       const { checkBatches, plantBatchMistake } = require('../src/testing/batch_check');
-      const one = (name, graph, keep) => {
-        const plain = lowerMI355X(graph, { perf: true, keep, batch: false, absorb: true });
-        const batched = lowerMI355X(graph, { perf: true, keep, absorb: true });
+      const one = (name, graph, keep, absorb = true) => {
+        const plain = lowerMI355X(graph, { perf: true, keep, batch: false, absorb });
+        const batched = lowerMI355X(graph, { perf: true, keep, absorb });
         const res = { name, launches: batched.launches.length, check: checkBatches(plain, batched),
           merged: (batched.batches || []).filter((b) => b.merged).map((b) => ({ count: b.count, kind: batched.launches[b.start].kind, kernel: b.kernels[0].name })) };
         if (req.plant) {
@@ -1450,7 +1450,7 @@ async function main() {
       }
       for (const c of req.graphs || []) {
         const f = fuse(Graph.fromJSON(c.graph), { keep: c.keep });
-        out.push(one(c.name, f.graph, c.keep.map((id) => f.index.get(id))));
+        out.push(one(c.name, f.graph, c.keep.map((id) => f.index.get(id)), false));
       }
       break;
     }

@@ -23,7 +23,7 @@ def test_merged_kernels_store_each_members_own_values(tool):
     res = {r["name"]: r for r in tool("batch-check", {"graphs": graphs(tool), "models": [{"model": "transformer", "B": 64, "attention": True}],
                                                       "plant": True})}
     assert all(r["check"]["ok"] for r in res.values()), [r for r in res.values() if not r["check"]["ok"]]
-    assert res["chain-0-8192x1024"]["merged"][0]["count"] >= 3 and res["chain-13-4097x515"]["merged"][0]["count"] == 2
+    assert res["chain-0-8192x1024"]["merged"][0]["count"] == 4 and res["chain-13-4097x515"]["merged"][0]["count"] == 2
     assert res["logSoftmax-16384x4096"]["merged"][0]["count"] == 2 and res["logSoftmax-4099x2049"]["merged"][0]["count"] == 2
     assert res["softmax-8193x61"]["merged"] and res["transformer-64-attention"]["merged"]
     # A grid that does not fill the chip keeps its members side by side.
