@@ -113,6 +113,29 @@ __device__ __forceinline__ float4 vop(float4 x) {
   else return x;
 }
 
+// A per-element (MODE_S) operand one of whose indices is contiguous all the same, its rows of a
+// length or at an offset that is no multiple of 4: V::RUN 1 names the column, 2 the row. It is
+// staged as MODE_C or MODE_R, by 128-bit loads of 4-byte alignment, single ones where a
+// group of 4 crosses the end of the run. (777 x 1000 x 515, both operands such: 20.9 us
+// against 34.2 with one load per element; 1000 x 777 x 515 20.3 against 28.1.)
+template <class V>
+__device__ constexpr auto view_run(int) -> decltype(V::RUN, int()) { return V::RUN; }
+template <class V>
+__device__ constexpr int view_run(long) { return 0; }
+template <int MODE, class V>
+__device__ constexpr int staged_mode() {
+  return MODE != MODE_S ? MODE : view_run<V>(0) == 1 ? static_cast<int>(MODE_C) : view_run<V>(0) == 2 ? static_cast<int>(MODE_R) : static_cast<int>(MODE_S);
+}
+typedef float run4 __attribute__((ext_vector_type(4), aligned(4)));
+// Four elements of a run at p, of which `left` (1 or more) are inside the operand; 0 past them.
+__device__ __forceinline__ float4 load_run4(const float* p, uint32_t left) {
+  if (left >= 4u) {
+    const run4 r = *reinterpret_cast<const run4*>(p);
+    return make_float4(r[0], r[1], r[2], r[3]);
+  }
+  return make_float4(p[0], left > 1u ? p[1] : 0.f, left > 2u ? p[2] : 0.f, 0.f);
+}
+
 // A workgroup's (x, y, z) place in its launch's grid.
 struct Wg {
   uint32_t x, y, z;
@@ -134,11 +157,11 @@ __device__ __forceinline__ Wg xcd_grouped() {
   return {t % gx, t / gx, L % 8u + 8u * (rest / G)};
 }
 
-// A staged tile's padded row stride and floats: As[row][k] or (MODE_R) As[k][row], Bs[k][col]
+// A staged tile's (of the operands' staged_mode) padded row stride and floats: As[row][k] or (MODE_R) As[k][row], Bs[k][col]
 // or (MODE_R) Bs[col][k].
-template <int BM, int BN, int BK, int AMODE, int BMODE>
+template <int BM, int BN, int BK, int AMODE, int BMODE, class AV, class BV>
 struct GemmTiles {
-  static constexpr bool A_KMAJOR = AMODE == MODE_R, B_NMAJOR = BMODE == MODE_R;
+  static constexpr bool A_KMAJOR = staged_mode<AMODE, AV>() == MODE_R, B_NMAJOR = staged_mode<BMODE, BV>() == MODE_R;
   static constexpr int AS = A_KMAJOR ? BM + 4 : BK + 4;
   static constexpr int BS = B_NMAJOR ? BK + 4 : BN + 4;
   static constexpr int A = (A_KMAJOR ? BK : BM) * AS, B = (B_NMAJOR ? BN : BK) * BS;
@@ -157,7 +180,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
   constexpr int BN = WN * TN * 16;
   static_assert(BK == 16 || BK == 32 || BK == 64, "slice depth");
   static_assert(PF == 1 || PF == 2, "prefetch depth");
-  using Tiles = GemmTiles<BM, BN, BK, AMODE, BMODE>;
+  using Tiles = GemmTiles<BM, BN, BK, AMODE, BMODE, AV, BV>;
   constexpr bool A_KMAJOR = Tiles::A_KMAJOR, B_NMAJOR = Tiles::B_NMAJOR;
   constexpr int AS = Tiles::AS, BS = Tiles::BS;
   float (*As)[Tiles::A] = reinterpret_cast<float (*)[Tiles::A]>(As_);
@@ -173,7 +196,8 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
   constexpr int B_VEC = (BK * BN / 4 + THREADS - 1) / THREADS;
   constexpr int A_SC = (BM * BK + THREADS - 1) / THREADS;        // scalar loads per thread
   constexpr int B_SC = (BK * BN + THREADS - 1) / THREADS;
-  constexpr bool VA = AMODE != MODE_S, VB = BMODE != MODE_S;
+  constexpr int AM = staged_mode<AMODE, AV>(), BMD = staged_mode<BMODE, BV>();
+  constexpr bool VA = AM != MODE_S, VB = BMD != MODE_S;
   // Staging registers for a slice in flight: one set, or two for PF = 2 (the
   // global loads of slice k + 2 are issued while slice k is computed, so each
   // load has two slices' compute to arrive before it is stored to LDS).
@@ -190,24 +214,28 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
     float4* rb = S.rb;
     float* sa = S.sa;
     float* sb = S.sb;
-    if (AMODE == MODE_C) {
+    if (AM == MODE_C) {
 #pragma unroll
       for (int v = 0; v < A_VEC; ++v) {
         const int t = tid + v * THREADS;
         const uint32_t row = t / (BK / 4), kk = (t % (BK / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (t < BM * BK / 4 && m0 + row < M && k0 + kk < kend)
-          x = *reinterpret_cast<const float4*>(Ab + vrow<AV>(m0 + row) + vcol<AV>(k0 + kk));
+        if (t < BM * BK / 4 && m0 + row < M && k0 + kk < kend) {
+          if constexpr (view_run<AV>(0) != 0) x = load_run4(Ab + vrow<AV>(m0 + row) + vcol<AV>(k0 + kk), kend - (k0 + kk));
+          else x = *reinterpret_cast<const float4*>(Ab + vrow<AV>(m0 + row) + vcol<AV>(k0 + kk));
+        }
         ra[v] = x;
       }
-    } else if (AMODE == MODE_R) {
+    } else if (AM == MODE_R) {
 #pragma unroll
       for (int v = 0; v < A_VEC; ++v) {
         const int t = tid + v * THREADS;
         const uint32_t kk = t / (BM / 4), row = (t % (BM / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (t < BM * BK / 4 && m0 + row < M && k0 + kk < kend)
-          x = *reinterpret_cast<const float4*>(Ab + vcol<AV>(k0 + kk) + vrow<AV>(m0 + row));
+        if (t < BM * BK / 4 && m0 + row < M && k0 + kk < kend) {
+          if constexpr (view_run<AV>(0) != 0) x = load_run4(Ab + vcol<AV>(k0 + kk) + vrow<AV>(m0 + row), M - (m0 + row));
+          else x = *reinterpret_cast<const float4*>(Ab + vcol<AV>(k0 + kk) + vrow<AV>(m0 + row));
+        }
         ra[v] = x;
       }
     } else {
@@ -220,24 +248,28 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         sa[v] = x;
       }
     }
-    if (BMODE == MODE_C) {
+    if (BMD == MODE_C) {
 #pragma unroll
       for (int v = 0; v < B_VEC; ++v) {
         const int t = tid + v * THREADS;
         const uint32_t kk = t / (BN / 4), c = (t % (BN / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (t < BK * BN / 4 && k0 + kk < kend && n0 + c < N)
-          x = *reinterpret_cast<const float4*>(Bb + vrow<BV>(k0 + kk) + vcol<BV>(n0 + c));
+        if (t < BK * BN / 4 && k0 + kk < kend && n0 + c < N) {
+          if constexpr (view_run<BV>(0) != 0) x = load_run4(Bb + vrow<BV>(k0 + kk) + vcol<BV>(n0 + c), N - (n0 + c));
+          else x = *reinterpret_cast<const float4*>(Bb + vrow<BV>(k0 + kk) + vcol<BV>(n0 + c));
+        }
         rb[v] = x;
       }
-    } else if (BMODE == MODE_R) {
+    } else if (BMD == MODE_R) {
 #pragma unroll
       for (int v = 0; v < B_VEC; ++v) {
         const int t = tid + v * THREADS;
         const uint32_t c = t / (BK / 4), kk = (t % (BK / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (t < BK * BN / 4 && k0 + kk < kend && n0 + c < N)
-          x = *reinterpret_cast<const float4*>(Bb + vcol<BV>(n0 + c) + vrow<BV>(k0 + kk));
+        if (t < BK * BN / 4 && k0 + kk < kend && n0 + c < N) {
+          if constexpr (view_run<BV>(0) != 0) x = load_run4(Bb + vcol<BV>(n0 + c) + vrow<BV>(k0 + kk), kend - (k0 + kk));
+          else x = *reinterpret_cast<const float4*>(Bb + vcol<BV>(n0 + c) + vrow<BV>(k0 + kk));
+        }
         rb[v] = x;
       }
     } else {
@@ -257,7 +289,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
     const float4* rb = S.rb;
     const float* sa = S.sa;
     const float* sb = S.sb;
-    if (AMODE == MODE_C) {
+    if (AM == MODE_C) {
 #pragma unroll
       for (int v = 0; v < A_VEC; ++v) {
         const int t = tid + v * THREADS;
@@ -266,7 +298,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
           *reinterpret_cast<float4*>(&As[buf][row * AS + kk]) = vop<AV>(ra[v]);
         }
       }
-    } else if (AMODE == MODE_R) {
+    } else if (AM == MODE_R) {
 #pragma unroll
       for (int v = 0; v < A_VEC; ++v) {
         const int t = tid + v * THREADS;
@@ -282,7 +314,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         if (t < BM * BK) As[buf][(t / BK) * AS + (t % BK)] = vop<AV>(sa[v]);
       }
     }
-    if (BMODE == MODE_C) {
+    if (BMD == MODE_C) {
 #pragma unroll
       for (int v = 0; v < B_VEC; ++v) {
         const int t = tid + v * THREADS;
@@ -291,7 +323,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
           *reinterpret_cast<float4*>(&Bs[buf][kk * BS + c]) = vop<BV>(rb[v]);
         }
       }
-    } else if (BMODE == MODE_R) {
+    } else if (BMD == MODE_R) {
 #pragma unroll
       for (int v = 0; v < B_VEC; ++v) {
         const int t = tid + v * THREADS;
@@ -463,7 +495,7 @@ __device__ __forceinline__ void gemm_f32(const Args& A, const float* __restrict_
   constexpr int THREADS = 64 * 2 * WN;   // threads of one K group
   constexpr int BM = 2 * TM * 16;
   constexpr int BN = WN * TN * 16;
-  using Tiles = GemmTiles<BM, BN, BK, AMODE, BMODE>;
+  using Tiles = GemmTiles<BM, BN, BK, AMODE, BMODE, AV, BV>;
   // The tiles (and the K groups' hand-over area) live in one LDS pool of this size: two
   // instantiations of the same size in one kernel (members of one batched launch whose
   // operand views differ) share it instead of adding up.

@@ -216,7 +216,7 @@ __device__ __forceinline__ void gemm_bf16x3(const Args& A, const float* __restri
   using SA = Bf16x3Stage<AV, false, BM, THREADS, AKC, KT>;
   using SB = Bf16x3Stage<BV, true, BN, THREADS, BKC, KT>;
   constexpr int BUF = SA::BYTES + SB::BYTES;
-  using Tiles = GemmTiles<BM, BN, 16, AMODE, BMODE>;
+  using Tiles = GemmTiles<BM, BN, 16, AMODE, BMODE, AV, BV>;
   constexpr int FP32 = 4 * 2 * (Tiles::A + Tiles::B);
   constexpr int POOL = 2 * BUF > FP32 ? 2 * BUF : FP32;
   float* const pool = lds_pool<POOL / 4>();

@@ -859,13 +859,14 @@ const BF16X3_TILES = [{ tm: 4, tn: 4, wn: 4, cost: 1 }, { tm: 2, tn: 2, wn: 4, c
  * The tiling of a product on the bf16 matrix cores (tcmi_gemm_bf16x3.h), or null where the
  * fp32 kernel is the better one. Measured, fp32 against bf16 parts:
  *   4096^3 1040 against 620 us; 8192 x 256 x 1024 43 / 30.7; 8192 x 1024 x 256 43.4 / 34.8;
- *   8192 x 256 x 256 14.3 / 12.2; 1024^3 42.4 / 24.1; 1000 x 515 x 777 30 / 16.6;
+ *   8192 x 256 x 256 14.3 / 12.2; 1024^3 42.4 / 24.1; 1000 x 515 x 777 18.8 / 17.2;
  *   4 weight gradients 256 x 8192 x 1024 179 / 110, 16 of 256 x 8192 x 256 165 / 119.
  * fp32 keeps
  *   - products it sums in K groups (few tiles): 512^3 5.2 against 12.7 us, 640^3 12.2 / 17.3;
  *     K groups also leave it the smaller error (512^3 without its bias: 2.1e-7 against 3.4e-7);
  *   - a K below 96 (8192 x 96 x 256 8.8 / 7.9, 1024 x 64 x 1024 5.6 / 5.6), or below 512
- *     where the tiles do not fill the chip (768 x 256 x 768 7.9 / 9.1);
+ *     where the tiles do not fill the chip (768 x 256 x 768 7.9 / 9.1), and any K where they
+ *     leave a quarter of it idle (1000 x 777 x 515, 144 tiles, 20.3 / 25.5);
  *   - products that would pad by more than a fifth (8192 x 256 x 96 7.9 / 8.7).
  * Each CU runs its tiles one after another (the chip's 256 at a time), so the tile is the one
  * with the least rounds x area x cost. K is split no less than the fp32 kernel splits it (`chunks`:
@@ -883,7 +884,7 @@ function bf16x3Tiling(batch, M, N, K, peers, chunks) {
     const chunkK = Math.ceil(Math.ceil(K / parts) / 32) * 32;
     parts = Math.ceil(K / chunkK);
     const all = tiles * parts * (chunks === 1 ? 1 : peers);
-    if (all < 128 || (all < 256 && K < 512)) continue;
+    if (all < 192 || (all < 256 && K < 512)) continue;
     const cost = Math.ceil(all / 256) * bm * bn * c.cost * chunkK;
     if (!best || cost < best.cost) best = { cost, tm: c.tm, tn: c.tn, wn: c.wn, chunks: parts, chunkK, blocks: tiles * parts };
   }
@@ -893,7 +894,7 @@ function bf16x3Tiling(batch, M, N, K, peers, chunks) {
 
 /**
  * Floats of the LDS pool (tcmi::lds_pool) tcmi_gemm.h's gemm_f32 takes for tiling `tl`
- * and operand load modes (0 row-major, 1 transposed, 2 strided): both staged slices of
+ * and operand staging modes (0 row-major, 1 transposed, 2 strided): both staged slices of
  * each K group's A and B tiles, rows padded by 4, and the K groups' hand-over area.
  */
 function gemmPoolFloats(tl, amode, bmode) {
@@ -968,21 +969,24 @@ function operandView(name, view, batchDims, R, C) {
 };
 `;
     const span = (fs) => fs.reduce((t, [e, st]) => t + (e - 1) * st, 0);
-    return { text, mode, limit: 1 + batchLimit + span(rf) + span(cf), mapped: true, rows: mode === 1, cols: mode === 0 };
+    return { text, mode, limit: 1 + batchLimit + span(rf) + span(cf), mapped: true, rows: mode === 1, cols: mode === 0, staged: mode };
   }
   const others4 = (x) => strides.every((s) => s % 4 === 0) && x % 4 === 0;
   let mode = 2;
   if (v.sc === 1 && C % 4 === 0 && others4(v.sr)) mode = 0;
   else if (v.sr === 1 && R % 4 === 0 && others4(v.sc)) mode = 1;
+  // A per-element operand whose elements still lie in runs (tcmi_gemm.h view_run). Runs shorter than
+  // two tiles are mostly their ends: config 1's 128 x 128 x 10 product 4.1 us per element, 4.7 as runs.
+  const run = mode !== 2 ? 0 : v.sc === 1 && C >= 64 ? 1 : v.sr === 1 && R >= 64 ? 2 : 0;
   const text = `struct ${name} {
-  static constexpr size_t SR = ${v.sr}, SC = ${v.sc};${loadOp(v)}
+  static constexpr size_t SR = ${v.sr}, SC = ${v.sc};${loadOp(v)}${run ? `\n  static constexpr int RUN = ${run};` : ''}
   static __device__ __forceinline__ size_t batch(uint32_t b) { return ${batchTerms}; }
 };
 `;
   // One past the largest element offset the kernel can address.
   const limit = 1 + batchLimit + (R - 1) * v.sr + (C - 1) * v.sc;
   // rows, cols: whether that index is the contiguous one, whatever the alignment.
-  return { text, mode, limit, rows: v.sr === 1, cols: v.sc === 1 };
+  return { text, mode, limit, rows: v.sr === 1, cols: v.sc === 1, staged: run === 1 ? 0 : run === 2 ? 1 : mode };
 }
 
 /**
@@ -1084,7 +1088,7 @@ ${grouped ? `  ${XCD_GROUPED}
   const text = `#include "${tl.bf3 ? 'tcmi_gemm_bf16x3.h' : 'tcmi_gemm.h'}"\n${av.text}${bv.text}${epi}${main}`;
   const k = kernelText('mm', text);
   const kernels = [{ name: k.name, source: k.source, grid: [Math.ceil(N / (16 * tl.wn * tl.tn)), Math.ceil(M / (32 * tl.tm)), batch * tl.chunks],
-    block: [threads, 1, 1], lds: 0, pool: gemmPoolFloats(tl, av.mode, bv.mode) }];
+    block: [threads, 1, 1], lds: 0, pool: gemmPoolFloats(tl, av.staged, bv.staged) }];
   let workspace = 0;
   if (split) {
     // The reduction kernel shares the epilogue struct of the partial kernel's text.

@@ -17,7 +17,7 @@ PKG = pathlib.Path(__file__).resolve().parent.parent / "tensor-compiler-webgpu_a
 
 # (M, K, N): one past and one short of the 128 x 256, 64 x 128 and 64 x 64 tiles, K ending 1, 3
 # and 31 short of a slice of 32 and a group of 4, rows of odd length (unaligned 128-bit loads).
-RAGGED = [(1000, 777, 515), (1025, 513, 767), (1087, 515, 1024), (961, 545, 1026), (4095, 97, 1021)]
+RAGGED = [(2049, 1027, 1025), (1087, 1025, 2047), (1023, 1058, 2050), (1000, 515, 1777), (4095, 97, 1021)]
 
 
 def test_forward_and_both_transposed_products_within_budget(tmp_path, tool):
@@ -81,7 +81,7 @@ def product(tool, x, w):
         t.module_unload(mod)
 
 
-@pytest.mark.parametrize("batch,M,K,N", [(1, 768, 512, 768), (1, 4097, 96, 1024), (1, 256, 8192, 512), (3, 520, 530, 900), (1, 1024, 4096, 2048)])
+@pytest.mark.parametrize("batch,M,K,N", [(1, 1024, 512, 832), (1, 4097, 96, 1024), (1, 256, 8192, 512), (3, 520, 530, 900), (1, 1024, 4096, 2048)])
 def test_sums_are_no_less_exact_than_fp32_ones(tool, batch, M, K, N):
     """Every element within gamma(K) of float64's, and their 2-norm error within what an fp32 sum of K terms makes: K
     roundings of 2^-24 / sqrt(3) of the partial sum, whose square grows as k / K (K / 2 in all), and the result's own."""
@@ -102,13 +102,13 @@ def test_sums_are_no_less_exact_than_fp32_ones(tool, batch, M, K, N):
 def test_selection_returns_the_values_bit_for_bit(tool):
     """A product with the identity's first columns: the three parts sum back to the value. Values over
     60 binades, zeros of both signs."""
-    print("gpu step: selection 1024x544x640", flush=True)
+    print("gpu step: selection 1024x544x832", flush=True)
     rng = np.random.default_rng(5)
     x = (rng.standard_normal((1024, 544)) * 2.0 ** rng.integers(-30, 30, (1024, 544))).astype(np.float32)
     x[::7, ::5] = 0.0
-    y, text = product(tool, x, np.eye(544, 640, dtype=np.float32))
+    y, text = product(tool, x, np.eye(544, 832, dtype=np.float32))
     assert "gemm_bf16x3" in text
-    want = np.zeros((1024, 640), dtype=np.float32)
+    want = np.zeros((1024, 832), dtype=np.float32)
     want[:, :544] = x
     assert np.array_equal(y, want)
 
@@ -117,10 +117,10 @@ def test_selection_returns_the_values_bit_for_bit(tool):
 def test_values_the_parts_do_not_cover_take_the_fp32_sums(tool, what):
     """One such row (and one column) among ordinary ones: IEEE results where they are not finite, fp32's accuracy
     where they are."""
-    print(f"gpu step: 1024x512x640, {what}", flush=True)
+    print(f"gpu step: 1024x512x832, {what}", flush=True)
     rng = np.random.default_rng(9)
     x = rng.standard_normal((1024, 512)).astype(np.float32)
-    w = rng.standard_normal((512, 640)).astype(np.float32)
+    w = rng.standard_normal((512, 832)).astype(np.float32)
     if what == "infinite":
         x[130, 7], w[9, 300] = np.inf, -np.inf
     elif what == "nan":
