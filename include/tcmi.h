@@ -182,7 +182,7 @@ int tcmi_graph_launch(uint64_t graph);
  * submit (trainer-fused.js:59-81: write the batch, submit, read the loss back):
  * `count` host->device copies of bytes[i] from src[i] to the allocation dst[i]
  * (offset 0) on the library stream, small ones staged through pinned host
- * memory, then the replay of `graph`, then `out_bytes` from the device address
+ * memory (which a kernel reads, and writes a small result to), then the replay of `graph`, then `out_bytes` from the device address
  * `out_src` into host `out`, then a wait for all of it. Everything is checked
  * before anything is enqueued; the sources may be reused when it returns. */
 int tcmi_graph_step(uint32_t count, const uint64_t* dst, const void* const* src, const uint64_t* bytes, uint64_t graph,
