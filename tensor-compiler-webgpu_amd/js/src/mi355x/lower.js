@@ -1272,6 +1272,8 @@ function lowerOnce(graph, opts, noAbsorb, noForm) {
  *      grids, are grouped the same way (each window tried in turn as a group's
  *      first) into ragged batches (codegen.js raggedKernel): one dispatch of their
  *      summed workgroups, each member over its own range of them.
+ * A batch whose members read the same operands is then computed by one kernel (`merged`:
+ * codegen.js mergedKernel).
  * Every launch thus stays after its operands' writers and before its output's
  * readers, so it reads exactly the values it read in graph order, and writes its
  * own node's buffer (a batch's members each their own workspace slice). A batch
