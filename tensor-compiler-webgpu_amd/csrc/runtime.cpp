@@ -783,6 +783,14 @@ int tcmi_graph_step(uint32_t count, const uint64_t* dst, const void* const* src,
     if (!bytes[i]) continue;
     void* d = reinterpret_cast<void*>(dst[i]);
     const uint64_t b = bytes[i];
+    // Copies land in the call's order where they overlap: one that writes over a copy that waits
+    // for the kernel follows that kernel.
+    for (uint32_t k = 0; k < ups; ++k) {
+      const uint64_t at = reinterpret_cast<uint64_t>(up.dst[k]);
+      if (dst[i] >= at + 4ull * up.words[k] || at >= dst[i] + b) continue;
+      if ((e = enqueue_copies(up, ups, g_stream)) != hipSuccess) return drained(e, "k_copies launch (uploads)");
+      ups = 0;
+    }
     if (b <= (kStageBytes >> 2) && staged + b <= kStageBytes - 4096) {
       std::memcpy(g_stage + staged, src[i], b);
       if (b % 4 == 0 && dst[i] % 4 == 0 && ups < kMaxCopies) {

@@ -58,6 +58,48 @@ def test_graph_step_uploads_replays_and_reads_back():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("ranges", [
+    [(0, 64), (32, 64)],                                    # the second over the first's tail
+    [(0, 256), (16, 8), (20, 2), (0, 1)],                   # odd ones among them, over earlier ones
+    [(0, 1 << 10), (0, 1 << 20), (512, 1 << 10)],           # a direct one over a staged one, and back
+    [(24 * i, 40) for i in range(21)],                      # more than one kernel takes, each over the last
+    [(40 * i, 40) for i in range(21)],                      # and none over another
+], ids=["tail", "odd", "direct", "many", "apart"])
+def test_graph_step_uploads_land_in_order(ranges):
+    """Uploads of one step that overlap in the same buffer land in the call's order, in every mix
+    of the routes a copy may take; the step reads what the last one left."""
+    import tcmi_ctypes
+    t = tcmi_ctypes.load()
+    t.init()
+    u64 = tcmi_ctypes.u64
+    size, n = 1 << 21, len(ranges)
+    h, g = u64(), u64()
+    t.malloc(size, ctypes.byref(h))
+    try:
+        t.fill32(h.value, 0, 0, size // 4)
+        t.capture_begin()
+        t.fill32(h.value, size - 4, 7, 1)
+        t.capture_end(ctypes.byref(g))
+        want = np.zeros(size, dtype=np.uint8)
+        parts = [np.random.default_rng(i).integers(1, 255, b, dtype=np.uint8) for i, (_, b) in enumerate(ranges)]
+        for (at, b), part in zip(ranges, parts):
+            want[at:at + b] = part
+        want[-4:] = np.frombuffer(np.uint32(7).tobytes(), dtype=np.uint8)
+        dst = (u64 * n)(*[h.value + at for at, _ in ranges])
+        src = (ctypes.c_void_p * n)(*[part.ctypes.data for part in parts])
+        nbytes = (u64 * n)(*[b for _, b in ranges])
+        out = np.zeros(4, dtype=np.uint8)
+        assert t.lib.tcmi_graph_step(n, dst, src, nbytes, g.value, h.value + size - 4, out.ctypes.data, 4) == 0, t.lib.tcmi_last_error()
+        assert np.array_equal(out, want[-4:])
+        back = np.zeros(size, dtype=np.uint8)
+        t.d2h(back.ctypes.data, h.value, 0, size)
+        assert np.array_equal(back, want)
+        t.graph_destroy(g.value)
+    finally:
+        t.free(h.value)
+
+
+@pytest.mark.gpu
 def test_launch_dag_over_several_streams_is_refused_inside_a_capture():
     """Capture over several streams is switched off in the C ABI itself: an empty
     two-stream launch group is accepted eagerly and refused, with nothing enqueued,
