@@ -1414,6 +1414,11 @@ function batchPlan(launches, aliases, bytesOf) {
     const outs = total(u.map((l) => l.node));
     const apart = outs + u.reduce((q, l) => q + total(reads(l)), 0);
     if (5 * (outs + total([].concat(...u.map(reads)))) > 4 * apart) return null;
+    // Rows that a whole workgroup reduces: only where the batch moves 128 MiB or more, half of the
+    // last-level cache, which below that serves the second read (logSoftmax's gradient over
+    // [16384, 4096], 1.3 GB: 203 us apart, 172 merged; LayerNorm's over [2176, 960], under 60 MB:
+    // 16.5 apart, 17.5 merged).
+    if (apart < 2 ** 27 && u.some((l) => cg.mergeOnly(l.kernels[0]))) return null;
     return cg.mergedKernel(u.map((l) => ({ kernel: l.kernels[0], reads: reads(l) })));
   };
   const order = [], batches = [];
