@@ -38,6 +38,11 @@ function literal(v) {
   return `tcmi::f32_bits(0x${u32[0].toString(16).padStart(8, '0')}u)`;
 }
 
+/** `v` as text for a key: JSON, with the numbers that JSON writes alike (0 and -0; infinities and NaN) told apart. */
+function keyText(v) {
+  return JSON.stringify(v, (k, x) => (Object.is(x, -0) ? '-0' : typeof x === 'number' && !Number.isFinite(x) ? String(x) : x));
+}
+
 /** FNV-1a over a string, as 8 hex digits (kernel names). */
 function fnv(s) {
   let h = 0x811c9dc5;
@@ -1757,7 +1762,7 @@ function mergedKernel(members) {
         return;
       }
       const inputs = n.inputs.map((i) => at.get(i));
-      at.set(id, add(`${n.op} ${inputs} ${JSON.stringify(n.attrs)} ${n.shape}`, { op: n.op, inputs, attrs: n.attrs, shape: n.shape }));
+      at.set(id, add(`${n.op} ${inputs} ${keyText(n.attrs)} ${n.shape}`, { op: n.op, inputs, attrs: n.attrs, shape: n.shape }));
     });
     return { id: at.get(output), ptr: `B.m[${m}].out`, nt };
   });
@@ -1875,5 +1880,5 @@ ${branches.join('\n')}
 
 module.exports = { elementwiseKernel, rowwiseKernel, colreduceKernels, gemmKernel, gemmTiling, attentionKernel, attentionGradKernel,
   gradPart, GRAD_PARTS, classifyGather, gatherStrides,
-  literal, fnv, Emitter, ParamOverflow, WG, MAX_P, MAX_IN, MAX_BATCH, batchable, batchedKernel, batchFamily,
+  literal, keyText, fnv, Emitter, ParamOverflow, WG, MAX_P, MAX_IN, MAX_BATCH, batchable, batchedKernel, batchFamily,
   mergedKernel, mergeOnly, raggable, raggedFits, raggedKernel, textLds, RAGGED_MAX_BLOCKS, RAGGED_MAX_LDS, COLRED_ONE_PASS };

@@ -33,6 +33,23 @@ def test_merged_kernels_store_each_members_own_values(tool):
         assert not res[name]["body"]["ok"] and "member" in res[name]["body"]["why"], (name, res[name]["body"])
 
 
+def over_zeros():
+    """exp(x) / 0 and exp(x) / -0, one operand read by both: inf and -inf."""
+    shape = [8192, 1024]
+    n = [("input", [], {"name": "x", "shape": shape}, shape), ("exp", [0], {}, shape)]
+    for zero in (0.0, -0.0):
+        at = len(n)
+        n += [("const", [], {"shape": [], "value": zero}, []), ("broadcast", [at], {"shape": shape}, shape), ("div", [1, at + 1], {}, shape)]
+    return {"nodes": [{"id": i, "op": op, "inputs": ins, "attrs": attrs, "shape": s} for i, (op, ins, attrs, s) in enumerate(n)]}
+
+
+def test_constants_that_differ_in_their_sign_of_zero_stay_apart(tool):
+    """Two members that differ in a constant, 0 and -0: each output is its own member's."""
+    r = tool("batch-check", {"graphs": [{"name": "zeros", "graph": over_zeros(), "keep": [4, 7]}]})[0]
+    assert r["merged"] and r["merged"][0]["count"] == 2
+    assert r["check"]["ok"], r["check"]
+
+
 @pytest.mark.gpu
 def test_merged_chains_equal_the_plain_lowering(tmp_path, tool):
     import tcmi_bridge
