@@ -1202,7 +1202,7 @@ function lowerOnce(graph, opts, noAbsorb, noForm) {
     // Kernels depend on structure, shapes, operand views, folded broadcasts and last
     // reads only: reuse across identical nodes.
     const peers = peersOf(node);
-    const key = JSON.stringify([node.op, node.inputs.map((id) => graph.nodes[id].shape), node.attrs, node.shape,
+    const key = cg.keyText([node.op, node.inputs.map((id) => graph.nodes[id].shape), node.attrs, node.shape,
       node.op === 'fused' ? opts.sabotage : null, opts.tuning || null, mmViews, foldKey, rowKey, lastReads, peers, absorbKey, formKey,
       streamOut.get(node.id), colKey]);
     let k = cache.get(key);

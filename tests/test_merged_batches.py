@@ -50,6 +50,14 @@ def test_constants_that_differ_in_their_sign_of_zero_stay_apart(tool):
     assert r["check"]["ok"], r["check"]
 
 
+def test_launches_that_differ_in_their_sign_of_zero_run_their_own_kernels(tool):
+    """The same two nodes as launches of the plain lowering, which shares a kernel among nodes alike."""
+    res = tool("lower", {"graph": over_zeros(), "fuse": {"keep": [4, 7]}, "sources": True})
+    a, b = [x["kernels"][0] for x in res["launches"] if "op_div" in x["kernels"][0]["source"]]
+    assert "f32_bits(0x00000000u)" in a["source"] and "f32_bits(0x80000000u)" not in a["source"]
+    assert "f32_bits(0x80000000u)" in b["source"] and "f32_bits(0x00000000u)" not in b["source"]
+
+
 @pytest.mark.gpu
 def test_merged_chains_equal_the_plain_lowering(tmp_path, tool):
     import tcmi_bridge
