@@ -1,7 +1,7 @@
 // fp32 matmul on CDNA4's bf16 matrix cores, with a fused epilogue.
 //
 // The bf16 matrix cores run 16 times as many flops as the fp32 ones, and a float32
-// is the exact sum of three bf16 numbers: x = x0 + x1 + x2, x0 = bf16(x), x1 =
+// is, but for the range, the exact sum of three bf16 numbers: x = x0 + x1 + x2, x0 = bf16(x), x1 =
 // bf16(x - x0), x2 = x - x0 - x1 (8 + 8 + 8 significant bits; both differences are
 // exact). So a·b = Σ a_i·b_j, each a_i·b_j exact in float32, and this kernel sums the
 // six products with i + j <= 2 into fp32 accumulators. The three left out are below
@@ -12,12 +12,14 @@
 // accumulator 6 times in 32 k, the fp32 kernel 8 times or more. Measured without a bias, fp32
 // against this: 4096^3 1.1e-6 / 1.0e-6, K 256 2.9e-7 / 2.3e-7, K 64 1.4e-7 / 0.9e-7.
 //
-// Where the split does not hold, the fp32 kernel decides: a tile is computed again by
-// gemm_f32_sum, in the same workgroup, if a sum is not finite (an infinity or NaN among the
-// operands, an overflow, or a value that bf16 rounds to infinity), if an operand is 2^100 or more,
-// or if a nonzero sum is below 2^-110 of the largest operand B. Operands below 2^-110 have no
-// exact third part (bf16 ends at 2^-133), but what they lose, at most 2^-134·B a product, is
-// below a rounding of any sum that is kept.
+// bf16's range ends at 2^-133 and float32's at 2^-149, so operands are split times 2^24: the parts of
+// every finite float32 below 2^103, subnormal ones too, then hold all its bits, and the sums are
+// multiplied by 2^-48 at the end. (Exact, and 1 % faster than to look for operands whose parts
+// lose bits: 4096^3 640 us against 645, 8192 x 1024 x 4096 with its gradients 1054 / 1069; a look at each
+// operand's magnitude as it is split 652, 1107.) Where that overflows, the fp32 kernel decides: a
+// tile with a sum that is not finite (an infinity or NaN among the operands, one that the scale or
+// bf16's rounding makes infinite, a sum of 2^80 or more) is computed again by gemm_f32_sum, in the
+// same workgroup.
 //
 // Operands are tcmi_gemm.h's views. The thread that loads an operand element splits it, so
 // LDS holds three bf16 tiles per operand and every wavefront reads its fragments as they
@@ -77,11 +79,9 @@ struct Minus {
   __device__ __forceinline__ float less_lo(float x, bf16x2 p) const { return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, lo), p, x, false); }
   __device__ __forceinline__ float less_hi(float x, bf16x2 p) const { return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, hi), p, x, false); }
 };
-// max(m, |a|, |b|), a NaN ignored.
-__device__ __forceinline__ float max3_abs(float m, float a, float b) {
-  asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(m) : "v"(a), "v"(b));
-  return m;
-}
+// What operands are multiplied by before they are split, so that a float32's lowest bit, 2^-149,
+// is above bf16's least normal value.
+constexpr float SPLIT_SCALE = 0x1p24f;
 
 // The operand's line index (A: row, B: column) and its k index as element offsets.
 template <class V, bool B>
@@ -105,7 +105,6 @@ struct Bf16x3Stage {
   __amdgpu_buffer_rsrc_t buf;
   uint32_t at[UNITS];    // byte offset of the unit's line (and, unmapped, of its first k in a slice)
   float x[UNITS][8];     // the slice in flight
-  float most;            // largest magnitude met so far
   Minus minus;
 
   static __device__ __forceinline__ int unit_line(int u) { return KC ? u / 64 * 16 + u % 16 : u % L; }
@@ -113,7 +112,6 @@ struct Bf16x3Stage {
 
   __device__ __forceinline__ void begin(const float* p, uint32_t bytes, uint32_t line0, uint32_t lines, int tid) {
     buf = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(p), 0, static_cast<int>(bytes), 0x00020000);
-    most = 0.f;
 #pragma unroll
     for (int v = 0; v < UNITS; ++v) {
       const int u = tid + v * THREADS;
@@ -184,8 +182,7 @@ struct Bf16x3Stage {
     u4 p0, p1, p2;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float a = vop<V>(e[2 * i]), b = vop<V>(e[2 * i + 1]);
-      most = max3_abs(most, a, b);
+      const float a = vop<V>(e[2 * i]) * SPLIT_SCALE, b = vop<V>(e[2 * i + 1]) * SPLIT_SCALE;
       const bf16x2 q0 = bf16_pair(a, b);
       const float a1 = minus.less_lo(a, q0), b1 = minus.less_hi(b, q0);
       const bf16x2 q1 = bf16_pair(a1, b1);
@@ -354,28 +351,23 @@ __device__ __forceinline__ void gemm_bf16x3(const Args& A, const float* __restri
   }
   __syncthreads();
 
-  // A tile the split does not cover is summed again in fp32. `largest`: the largest magnitude among
-  // the operands of the tile.
+  // The scale taken out; a tile that holds a sum that is not finite is summed again in fp32.
   uint32_t* const seen = reinterpret_cast<uint32_t*>(pool);
-  if (tid < 2) seen[tid] = 0u;
+  if (tid == 0) *seen = 0u;
   __syncthreads();
-  const float own = wave_reduce<true>(fmaxf(sa.most, sb.most));
-  if (lane == 0) atomicMax(seen, __float_as_uint(own));
-  __syncthreads();
-  const float largest = __uint_as_float(seen[0]);
-  bool again = !(largest < 0x1p100f);
+  float zero = 0.f;   // NaN after a sum that is not finite
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        const float v = fabsf(acc[i][j][r]);
-        again |= !(v < TCMI_INF) || (v < largest * 0x1p-110f && v != 0.f);
+        zero = fmaf(acc[i][j][r], 0.f, zero);
+        acc[i][j][r] *= 1.f / (SPLIT_SCALE * SPLIT_SCALE);
       }
-  if (again) seen[1] = 1u;
+  if (!(zero == 0.f)) *seen = 1u;
   __syncthreads();
-  const bool redo = __builtin_amdgcn_readfirstlane(seen[1]) != 0u;
+  const bool redo = __builtin_amdgcn_readfirstlane(*seen) != 0u;
   if (redo) {
     __syncthreads();
     gemm_f32_sum<TM, TN, 16, 1, AMODE, BMODE, AV, BV, WN, false>(pool, pool + 2 * Tiles::A, a_ptr + AV::batch(bz), b_ptr + BV::batch(bz), M,

@@ -151,7 +151,40 @@ def test_values_the_parts_do_not_cover_take_the_fp32_sums(tool, what):
     budget = 512 * 2.0 ** -24 * (np.abs(np.nan_to_num(x, posinf=0, neginf=0)).astype(np.float64)
                                  @ np.abs(np.nan_to_num(w, posinf=0, neginf=0)).astype(np.float64)) + 2.0 ** -126
     assert np.all(np.abs(y[finite] - exact[finite]) <= budget[finite])
-    if what in ("tiny", "wide"):   # 1e-35 has no third part in bf16; fp32 keeps all its bits
-        # (a row of 1e-32 keeps them too): 2-norm errors as an ordinary row's
+    if what in ("tiny", "wide"):   # 1e-35 by itself has no third part in bf16: 2-norm errors as an ordinary row's
         for r in (130, 500) if what == "tiny" else (130,):
             assert np.linalg.norm(y[r] - exact[r]) <= 1e-6 * np.linalg.norm(exact[r]), r
+
+
+@pytest.mark.parametrize("what,value,scale", [
+    ("no part in bf16", 2.0 ** -135, 2.0 ** 40), ("the least subnormal", 2.0 ** -149, 2.0 ** 90),
+    ("leading parts that cancel", 0.0, 2.0 ** 30)])
+def test_operands_below_the_range_of_bf16_keep_their_bits(tool, what, value, scale):
+    """An operand below 2^-134 is 0 in bf16, and a sum whose leading parts cancel is left with bits below bf16's range: a
+    sum of 0 if they are lost, an ordinary value in fp32, exact here (few bits)."""
+    print(f"gpu step: 1024x512x832, {what}", flush=True)
+    rng = np.random.default_rng(3)
+    x = rng.standard_normal((1024, 512)).astype(np.float32)
+    w = rng.standard_normal((512, 832)).astype(np.float32)
+    w[:, 300] = scale
+    if value:
+        x[130, :] = value
+    else:
+        x[130, :] = 0.0
+        x[130, 7], x[130, 300] = 2.0 ** -118 * (1 + 2.0 ** -20), -2.0 ** -118
+    y, text = product(tool, x, w)
+    assert "gemm_bf16x3" in text
+    assert y[130, 300] == (512 * value * scale if value else 2.0 ** -138 * scale)
+
+
+def test_subnormal_parts_keep_their_bits(tool):
+    """Operands whose third (below: second) part is subnormal as a bf16 by itself: exact, as every partial sum is a float32."""
+    print("gpu step: 1024x512x832, subnormal third parts", flush=True)
+    x = np.full((1024, 512), 2.0 ** -110 * (1 + 2.0 ** -9 + 2.0 ** -18), dtype=np.float32)
+    y, text = product(tool, x, np.ones((512, 832), dtype=np.float32))
+    assert "gemm_bf16x3" in text
+    assert np.all(y == np.float32(512 * 2.0 ** -110 * (1 + 2.0 ** -9 + 2.0 ** -18)))
+    # The second part, beside larger operands.
+    x[:, :256], x[:, 256:] = 2.0 ** -118 * (1 + 2.0 ** -9), 2.0 ** -108
+    y, _ = product(tool, x, np.ones((512, 832), dtype=np.float32))
+    assert np.all(y == np.float32(256 * (2.0 ** -118 + 2.0 ** -127 + 2.0 ** -108)))
