@@ -4,9 +4,9 @@
 // is, but for the range, the exact sum of three bf16 numbers: x = x0 + x1 + x2, x0 = bf16(x), x1 =
 // bf16(x - x0), x2 = x - x0 - x1 (8 + 8 + 8 significant bits; both differences are
 // exact). So a·b = Σ a_i·b_j, each a_i·b_j exact in float32, and this kernel sums the
-// six products with i + j <= 2 into fp32 accumulators. The three left out are below
-// 2^-26·|a·b| together, a quarter of one rounding of a float32 product. Six MFMAs take
-// 6/16 of the fp32 instructions' time.
+// six products with i + j <= 2 into fp32 accumulators. The three left out are at
+// most 2^-24·|a·b| together, one rounding of a float32 product (a = b = 1 + 2^-8 - 2^-17; over
+// normal values 2^-27.4 in the root mean square). Six MFMAs take 6/16 of the fp32 instructions' time.
 //
 // Error against float64 is no larger than the fp32 kernel's (tcmi_gemm.h): it rounds an
 // accumulator 6 times in 32 k, the fp32 kernel 8 times or more. Measured without a bias, fp32
@@ -294,8 +294,8 @@ __device__ __forceinline__ void gemm_bf16x3(const Args& A, const float* __restri
         __syncthreads();
         b_frags(to, 0, bn);
       }
-      // A column's six products from 0, the largest last, then one addition to the sums: an
-      // accumulator rounds once in 32 k. B first, A second: lane (t16, q) holds row t16,
+      // A column's six products are added to the sums in turn, the largest last: an accumulator
+      // rounds 6 times in 32 k. B first, A second: lane (t16, q) holds row t16,
       // columns 4q .. 4q+3.
       constexpr int PA[6] = {2, 1, 1, 0, 0, 0}, PB[6] = {0, 1, 0, 2, 1, 0};
 #pragma unroll

@@ -188,3 +188,14 @@ def test_subnormal_parts_keep_their_bits(tool):
     x[:, :256], x[:, 256:] = 2.0 ** -118 * (1 + 2.0 ** -9), 2.0 ** -108
     y, _ = product(tool, x, np.ones((512, 832), dtype=np.float32))
     assert np.all(y == np.float32(256 * (2.0 ** -118 + 2.0 ** -127 + 2.0 ** -108)))
+
+
+def test_products_left_out_add_to_no_more_than_a_rounding(tool):
+    """Operands of one value whose left-out products are the largest there are, all of one sign: 2^-24 of the sum. The
+    accumulator's roundings, 6 in 32 k, add at most 6 · (1 + .. + 16) / 16 = 51 of the result's."""
+    print("gpu step: 1024x512x832, the largest left-out products", flush=True)
+    c = np.float32(1 + 2.0 ** -8 - 2.0 ** -17)
+    y, text = product(tool, np.full((1024, 512), c), np.full((512, 832), c))
+    assert "gemm_bf16x3" in text
+    exact = 512 * float(c) ** 2
+    assert np.all(np.abs(y.astype(np.float64) - exact) <= (1 + 51) * 2.0 ** -24 * 1.001 * exact)
