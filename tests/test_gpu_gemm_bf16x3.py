@@ -38,15 +38,40 @@ def test_forward_and_both_transposed_products_within_budget(tmp_path, tool):
             assert j["pass"], (c["name"], s["slice"], j["first"], j["unjudged"])
 
 
-def product(tool, x, w):
-    """x [.., M, K] times w [.., K, N] by the plain lowering's kernels, in this process; and their text."""
+def operand(nodes, name, x, view):
+    """Appends the operand's nodes, reading `x` in place through `view`: 't' its last two axes exchanged,
+    'h' its axes [B, H, rows, cols] from [B, rows, H, cols], ('m', B, H) its [B·T, H·d] from [B, H, T, d].
+    Returns its node and the array the input holds."""
+    def add(op, ins, attrs, shape):
+        nodes.append({"op": op, "inputs": ins, "attrs": attrs, "shape": list(shape)})
+        return len(nodes) - 1
+
+    if view is None:
+        return add("input", [], {"name": name, "shape": list(x.shape)}, x.shape), x
+    perm = list(range(x.ndim - 2)) + [x.ndim - 1, x.ndim - 2] if view == "t" else [0, 2, 1, 3]
+    if view in ("t", "h"):
+        source, shape = x.transpose(perm), x.shape
+    else:
+        _, B, H = view
+        T, d = x.shape[0] // B, x.shape[1] // H
+        source, shape = x.reshape(B, T, H, d).transpose(perm), (B, T, H, d)
+    at = add("transpose", [add("input", [], {"name": name, "shape": list(source.shape)}, source.shape)], {"perm": perm}, shape)
+    return at if shape == x.shape else add("reshape", [at], {"shape": list(x.shape)}, x.shape), np.ascontiguousarray(source)
+
+
+def product(tool, x, w, views=(None, None)):
+    """x [.., M, K] times w [.., K, N], the operands behind `views`, by the lowering's kernels, in this process; and their text."""
     import tcmi_ctypes
     u32, u64 = tcmi_ctypes.u32, tcmi_ctypes.u64
     shape = list(x.shape[:-1]) + [w.shape[-1]]
-    graph = {"nodes": [{"op": "input", "inputs": [], "attrs": {"name": "x", "shape": list(x.shape)}, "shape": list(x.shape)},
-                       {"op": "input", "inputs": [], "attrs": {"name": "w", "shape": list(w.shape)}, "shape": list(w.shape)},
-                       {"op": "matmul", "inputs": [0, 1], "attrs": {}, "shape": shape}]}
-    launch = tool("lower", {"graph": graph, "sources": True})["launches"][0]
+    nodes = []
+    (a, x), (b, w) = operand(nodes, "x", x, views[0]), operand(nodes, "w", w, views[1])
+    nodes.append({"op": "matmul", "inputs": [a, b], "attrs": {}, "shape": shape})
+    res = tool("lower", {"graph": {"nodes": nodes}, "sources": True, "perf": True, "keep": [len(nodes) - 1]})["launches"]
+    assert len(res) == 1, "an operand is not read in place"
+    launch = res[0]
+    read = {i: v for i, v in zip([i for i, n in enumerate(nodes) if n["op"] == "input"], (x, w))}
+    x, w = (read[i] for i in launch["inputs"])
     t = tcmi_ctypes.load()
     t.init()
     t.set_include_dir(str(PKG / "csrc" / "kernels").encode())
@@ -66,7 +91,7 @@ def product(tool, x, w):
         y = np.empty(shape, dtype=np.float32)
         hx, hw, hy, ws = alloc(x.nbytes), alloc(w.nbytes), alloc(y.nbytes), alloc(max(16, launch["workspace"]))
         for h, v in ((hx, x), (hw, w)):
-            t.h2d(h, 0, np.ascontiguousarray(v).ctypes.data, v.nbytes)
+            t.h2d(h, 0, v.ctypes.data, v.nbytes)
         a = pack([hx, hw], hy, ws, launch["params"])
         for k in launch["kernels"]:
             f = u64()
@@ -199,3 +224,43 @@ def test_products_left_out_add_to_no_more_than_a_rounding(tool):
     assert "gemm_bf16x3" in text
     exact = 512 * float(c) ** 2
     assert np.all(np.abs(y.astype(np.float64) - exact) <= (1 + 51) * 2.0 ** -24 * 1.001 * exact)
+
+
+# Tiles (wavefronts along n, 16-wide tiles of one along m and n), views and what else sets an instantiation apart.
+FALLBACKS = [
+    ("128 x 256, transposed x", "<2, 4, 4, 4, false, false, false, 1, 0, false", (), 4096, 512, 4096, ("t", None)),
+    ("128 x 256, transposed w", "<2, 4, 4, 4, true, true, false, 0, 1, false", (), 1024, 256, 8192, (None, "t")),
+    ("64 x 128, both transposed", "<2, 4, 2, 2, false, true, false, 1, 1, false", (), 8192, 512, 256, ("t", "t")),
+    ("64 x 128, K split", "<2, 4, 2, 2, false, false, false, 1, 0, true", (), 256, 8192, 512, ("t", None)),
+    ("64 x 64, odd rows", "<2, 2, 2, 2, true, false, true, 2, 2, false", (), 1023, 513, 2049, (None, None)),
+    ("64 x 64, odd rows transposed", "<2, 2, 2, 2, false, true, true, 2, 2, false", (), 1023, 513, 2049, ("t", "t")),
+    ("64 x 64, batches", "<2, 2, 2, 2, true, false, true, 2, 0, false", (3,), 520, 530, 900, (None, None)),
+    ("64 x 128, heads", "<2, 4, 2, 2, true, false, false, 0, 0, false", (4, 2), 512, 128, 512, ("h", "h")),
+    ("64 x 128, mapped rows", "<2, 4, 2, 2, true, false, false, 0, 0, false", (), 2048, 512, 1024, (("m", 16, 4), None)),
+]
+
+
+@pytest.mark.parametrize("name,tile,lead,M,K,N,views", FALLBACKS, ids=[f[0] for f in FALLBACKS])
+def test_every_instantiation_falls_back(tool, name, tile, lead, M, K, N, views):
+    """One infinity in each operand, a NaN, a value that bf16 rounds to infinity, and a subnormal row in the last tile
+    against a large column there: IEEE results where they are not finite, fp32's accuracy where they are."""
+    print(f"gpu step: fallback, {name}", flush=True)
+    rng = np.random.default_rng(M + N)
+    x = rng.standard_normal(lead + (M, K)).astype(np.float32)
+    w = rng.standard_normal(lead + (K, N)).astype(np.float32)
+    w[..., K - 2, :] = np.where(np.abs(w[..., K - 2, :]) < 0.9, w[..., K - 2, :], 0.5)
+    x[..., M // 2, :], x[..., M // 2, K - 2] = 0.0, 3.4028235e38
+    x[..., 1, 7], w[..., 9, 3], x[..., M // 4, K - 1] = np.inf, -np.inf, np.nan
+    x[..., M - 1, :] = (rng.integers(1, 1 << 10, lead + (K,)) * 2.0 ** -149).astype(np.float32)
+    w[..., :, N - 1] *= np.float32(1e27)
+    y, text = product(tool, x, w, views)
+    assert "gemm_bf16x3" + tile in text
+    with np.errstate(invalid="ignore", over="ignore"):
+        exact = x.astype(np.float64) @ w.astype(np.float64)
+        want = exact.astype(np.float32)
+    finite = np.isfinite(want)
+    assert np.array_equal(np.isnan(y), np.isnan(want))
+    assert np.array_equal(y[~finite & ~np.isnan(want)], want[~finite & ~np.isnan(want)])
+    xs, ws = (np.abs(np.nan_to_num(v, nan=0.0, posinf=0.0, neginf=0.0)).astype(np.float64) for v in (x, w))
+    budget = K * 2.0 ** -24 * (xs @ ws) + 2.0 ** -126     # K roundings of products and partial sums; a subnormal may be flushed
+    assert np.all(np.abs(y[finite] - exact[finite]) <= budget[finite])
