@@ -1610,8 +1610,8 @@ function batchable(k, count) {
 /** The statement that opens a kernel whose workgroups take XCD-grouped places. */
 const XCD_GROUPED = 'const tcmi::Wg wg = tcmi::xcd_grouped();';
 
-/** Whether kernel `k` may only run in a batch that computes its members together (mergedKernel). */
-function mergeOnly(k) { return /^tcmi_row_[0-9a-f]+$/.test(k.name) && !!k.merge && /__shared__/.test(k.source); }
+/** Whether kernel `k` reduces each row across a workgroup (rowwise, with LDS). */
+function wideRows(k) { return /^tcmi_row_[0-9a-f]+$/.test(k.name) && /__shared__/.test(k.source); }
 
 /**
  * The family of kernel `k` for batching: its text with its operand view structs taken out
@@ -1628,9 +1628,6 @@ function batchFamily(k) {
   if (/^tcmi_row_[0-9a-f]+$/.test(k.name) && !k.lds && !k.ldsStatic && !/__shared__/.test(k.source)) {
     return `row@${k.grid.join(',')}/${k.block.join(',')}`;
   }
-  // Rowwise kernels that reduce a row across a workgroup fill the chip each: they are grouped
-  // only to be computed together (mergedKernel).
-  if (mergeOnly(k)) return `rows@${k.grid.join(',')}/${k.block.join(',')}`;
   // Matmul tiles take their LDS from a pool shared by instantiations of one size
   // (tcmi::lds_pool); other kernels' views would each add their own LDS: one text a family.
   if (!/^tcmi_mm_[0-9a-f]+$/.test(k.name)) return `${k.name}@${k.grid.join(',')}/${k.block.join(',')}/${k.lds}`;
@@ -1717,6 +1714,17 @@ const MERGED_MAX_MEMBERS = 8;
 const MERGED_MAX_HELD = 64;
 
 /**
+ * What members of one merged batch have in common, or null: elementwise kernels over one grid, rowwise
+ * ones that reduce within wavefronts, or rowwise ones that reduce across a workgroup. The
+ * last do not run side by side in a dispatch unless their texts are alike (batchFamily) or few (ragged
+ * batches), so they are grouped to be merged, and only as far as they can be.
+ */
+function mergeFamily(k) {
+  if (!k.merge) return null;
+  return wideRows(k) ? `rows@${k.grid.join(',')}/${k.block.join(',')}` : /^(ew|row)@/.test(batchFamily(k)) ? batchFamily(k) : null;
+}
+
+/**
  * The kernel of a merged batch: independent one-kernel launches over one grid and the same elements
  * (rows), all elementwise or all rowwise, whose bodies one kernel computes
  * together, storing each member's output. Each value is formed once, by the ops of its own
@@ -1733,10 +1741,10 @@ const MERGED_MAX_HELD = 64;
  */
 function mergedKernel(members) {
   const first = members[0].kernel, g = first.merge;
-  const family = batchFamily(first);
-  if (members.length < 2 || members.length > MERGED_MAX_MEMBERS || !/^(ew|rows?)@/.test(family) || first.grid[0] < MERGED_MIN_BLOCKS) return null;
+  const family = mergeFamily(first);
+  if (members.length < 2 || members.length > MERGED_MAX_MEMBERS || !family || first.grid[0] < MERGED_MIN_BLOCKS) return null;
   const like = (m) => JSON.stringify([m.rows || size(m.shape), m.tuning || null]);
-  if (!members.every(({ kernel: k }) => k.merge && !k.merge.sabotage && batchFamily(k) === family && like(k.merge) === like(g))) return null;
+  if (!members.every(({ kernel: k }) => mergeFamily(k) === family && !k.merge.sabotage && like(k.merge) === like(g))) return null;
   const nodes = [], known = new Map(), places = [];
   const streamed = new Set();
   const add = (key, node) => {
@@ -1881,4 +1889,4 @@ ${branches.join('\n')}
 module.exports = { elementwiseKernel, rowwiseKernel, colreduceKernels, gemmKernel, gemmTiling, attentionKernel, attentionGradKernel,
   gradPart, GRAD_PARTS, classifyGather, gatherStrides,
   literal, keyText, fnv, Emitter, ParamOverflow, WG, MAX_P, MAX_IN, MAX_BATCH, batchable, batchedKernel, batchFamily,
-  mergedKernel, mergeOnly, raggable, raggedFits, raggedKernel, textLds, RAGGED_MAX_BLOCKS, RAGGED_MAX_LDS, COLRED_ONE_PASS };
+  mergedKernel, mergeFamily, wideRows, raggable, raggedFits, raggedKernel, textLds, RAGGED_MAX_BLOCKS, RAGGED_MAX_LDS, COLRED_ONE_PASS };

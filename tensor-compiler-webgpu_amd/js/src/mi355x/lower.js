@@ -1273,7 +1273,8 @@ function lowerOnce(graph, opts, noAbsorb, noForm) {
  *      first) into ragged batches (codegen.js raggedKernel): one dispatch of their
  *      summed workgroups, each member over its own range of them.
  * A batch whose members read the same operands is then computed by one kernel (`merged`:
- * codegen.js mergedKernel).
+ * codegen.js mergedKernel). Launches of rows that a workgroup reduces do not share a dispatch by
+ * their grid alone: the first two passes group them only as far as they merge.
  * Every launch thus stays after its operands' writers and before its output's
  * readers, so it reads exactly the values it read in graph order, and writes its
  * own node's buffer (a batch's members each their own workspace slice). A batch
@@ -1294,6 +1295,24 @@ function batchPlan(launches, aliases, bytesOf) {
   // may share a dispatch.
   const one = (l) => (l.kernels.every((k) => cg.batchable(k)) ? l.kernels.map((k) => cg.batchFamily(k)).join(' ') : null);
   const fits = (l, count) => l.kernels.every((k) => cg.batchable(k, count));
+  // Members that read the same operands are computed together, each operand loaded once (codegen.js
+  // mergedKernel), where that takes a fifth or more off the bytes the batch moves.
+  const merged = (u) => {
+    if (!bytesOf || u.ragged || u.some((l) => l.kernels.length !== 1 || l.workspace)) return null;
+    const total = (ids) => Array.from(new Set(ids)).reduce((q, id) => q + bytesOf(id), 0);
+    const reads = (l) => l.inputs.map(owner);
+    const outs = total(u.map((l) => l.node));
+    const apart = outs + u.reduce((q, l) => q + total(reads(l)), 0);
+    if (5 * (outs + total([].concat(...u.map(reads)))) > 4 * apart) return null;
+    // Rows that a whole workgroup reduces: only where the batch moves 128 MiB or more, half of the
+    // last-level cache, which below that serves the second read (logSoftmax's gradient over
+    // [16384, 4096], 1.3 GB: 203 us apart, 172 merged; LayerNorm's over [2176, 960], under 60 MB:
+    // 16.5 apart, 17.5 merged).
+    if (apart < 2 ** 27 && cg.wideRows(u[0].kernels[0])) return null;
+    return cg.mergedKernel(u.map((l) => ({ kernel: l.kernels[0], reads: reads(l) })));
+  };
+  // Launches of rows that a workgroup reduces are grouped only where they merge.
+  const wide = (l) => (l.kernels.length === 1 && cg.wideRows(l.kernels[0]) ? cg.mergeFamily(l.kernels[0]) : null);
   // Pass 1: units (arrays of launches; two or more: a batch), in order.
   const placed = new Uint8Array(n);
   const ready = (l) => l.inputs.every((id) => { const w = writer.get(owner(id)); return w === undefined || placed[w] === 1; });
@@ -1323,9 +1342,16 @@ function batchPlan(launches, aliases, bytesOf) {
         continue;
       }
     }
-    const group = [i];
-    const name = one(launches[i]);
-    if (name) {
+    let group = [i];
+    const name = one(launches[i]), wideName = wide(launches[i]);
+    if (wideName) {
+      const like = [i];
+      for (let j = i + 1; j < n; j++) if (!placed[j] && wide(launches[j]) === wideName && ready(launches[j])) like.push(j);
+      const merges = (js) => merged(js.map((j) => launches[j]));
+      if (like.length > 1 && merges(like)) group = like;
+      else for (const j of like.slice(1)) if (merges(group.concat([j]))) group.push(j);
+    }
+    if (name && group.length === 1) {
       for (let j = i + 1; j < n && group.length < cg.MAX_BATCH; j++) {
         if (!placed[j] && one(launches[j]) === name && ready(launches[j])) group.push(j);
       }
@@ -1400,27 +1426,12 @@ function batchPlan(launches, aliases, bytesOf) {
       }
     }
   };
+  byWindows(wide, (group, l) => !!merged(group.concat([l])), null, true);
   byWindows(one, () => true, null, false);
   // Pass 3 (ragged batches): single-kernel launches of any kernels that may share a
   // dispatch whose members' grids differ (codegen.js raggedKernel) and still stand alone.
   const raggedKey = (l) => (l.kernels.length === 1 && !l.workspace && cg.raggable(l.kernels[0]) ? `ragged@${l.kernels[0].block[0]}` : null);
   byWindows(raggedKey, (group, l) => cg.raggedFits(group.concat([l]).map((m) => m.kernels[0])), (members) => { members.ragged = true; }, true);
-  // Members that read the same operands are computed together, each operand loaded once (codegen.js
-  // mergedKernel), where that takes a fifth or more off the bytes the batch moves.
-  const merged = (u) => {
-    if (!bytesOf || u.ragged || u.some((l) => l.kernels.length !== 1 || l.workspace)) return null;
-    const total = (ids) => Array.from(new Set(ids)).reduce((q, id) => q + bytesOf(id), 0);
-    const reads = (l) => l.inputs.map(owner);
-    const outs = total(u.map((l) => l.node));
-    const apart = outs + u.reduce((q, l) => q + total(reads(l)), 0);
-    if (5 * (outs + total([].concat(...u.map(reads)))) > 4 * apart) return null;
-    // Rows that a whole workgroup reduces: only where the batch moves 128 MiB or more, half of the
-    // last-level cache, which below that serves the second read (logSoftmax's gradient over
-    // [16384, 4096], 1.3 GB: 203 us apart, 172 merged; LayerNorm's over [2176, 960], under 60 MB:
-    // 16.5 apart, 17.5 merged).
-    if (apart < 2 ** 27 && u.some((l) => cg.mergeOnly(l.kernels[0]))) return null;
-    return cg.mergedKernel(u.map((l) => ({ kernel: l.kernels[0], reads: reads(l) })));
-  };
   const order = [], batches = [];
   for (const u of units) {
     if (u.joint) {
@@ -1433,8 +1444,6 @@ function batchPlan(launches, aliases, bytesOf) {
     const one = u.length > 1 ? merged(u) : null;
     if (one) {
       batches.push({ start: order.length, count: u.length, kernels: [one], wsStride: 0, merged: true });
-    } else if (u.length > 1 && u[0].kernels.some(cg.mergeOnly)) {
-      // Launches that gain nothing side by side: each by itself, in this order.
     } else if (u.length > 1 && u.ragged) {
       batches.push({ start: order.length, count: u.length, kernels: [cg.raggedKernel(u.map((m) => m.kernels[0]))], wsStride: 0, ragged: true });
     } else if (u.length > 1) {

@@ -33,6 +33,38 @@ def test_merged_kernels_store_each_members_own_values(tool):
         assert not res[name]["body"]["ok"] and "member" in res[name]["body"]["why"], (name, res[name]["body"])
 
 
+def copies(c, n):
+    """n independent copies of a graph, each over inputs of its own."""
+    nodes, keep = [], []
+    for i in range(n):
+        at = len(nodes)
+        for x in c["graph"]["nodes"]:
+            attrs = dict(x["attrs"], name=f"{x['attrs']['name']}{i}") if x["op"] == "input" else x["attrs"]
+            nodes.append(dict(x, inputs=[at + k for k in x["inputs"]], attrs=attrs))
+        keep += [at + k for k in c["keep"]]
+    return {"graph": {"nodes": nodes}, "keep": keep}
+
+
+def test_wide_rows_that_do_not_merge_share_dispatches_as_other_launches_do(tool):
+    """Rows that a workgroup reduces (2048 elements or more): few rows' launches in a ragged batch, launches of one text side
+    by side, a pair that reads one operand merged whatever else is ready beside it."""
+    few = [("softmax", 64, 4096), ("logSoftmax", 64, 4096), ("softmax", 256, 4096), ("logSoftmax", 512, 2048), ("softmax", 300, 3000)]
+    many = [("softmax", 64, 2048, 6, 1), ("softmax", 256, 2048, 3, 2), ("softmax", 16384, 4096, 6, 2), ("logSoftmax", 512, 2048, 4, 2)]
+    g = tool("config-graphs", {"c3": [{"fn": f, "R": R, "C": C} for f, R, C in few] + [{"fn": f, "R": R, "C": C} for f, R, C, _, _ in many]
+                               + [{"fn": "softmax", "R": 16384, "C": 4096}]})["c3"]
+    req = [dict(x["gradient"], name=f"one {x['fn']} {x['R']}x{x['C']}") for x in g[:len(few)]]
+    req += [dict(copies(x["forward"], m[3]), name=f"{m[3]} {x['fn']} {x['R']}x{x['C']}") for x, m in zip(g[len(few):], many)]
+    pair = g[-1]["gradient"], copies(g[-1]["forward"], 1)
+    n = len(pair[0]["graph"]["nodes"])
+    req.append({"name": "pair and another", "keep": pair[0]["keep"] + [n + k for k in pair[1]["keep"]], "graph": {"nodes": pair[0]["graph"]["nodes"]
+                + [dict(x, inputs=[n + k for k in x["inputs"]]) for x in pair[1]["graph"]["nodes"]]}})
+    res = tool("batch-check", {"graphs": req})
+    assert all(r["check"]["ok"] for r in res), [r for r in res if not r["check"]["ok"]]
+    dispatches = {r["name"]: r["launches"] - r["check"]["saved"] for r in res}
+    assert [dispatches[x["name"]] for x in req] == [1] * len(few) + [m[4] for m in many] + [2], dispatches
+    assert [r["merged"] for r in res[:-1]] == [[]] * (len(res) - 1) and res[-1]["merged"][0]["count"] == 2
+
+
 def over_zeros():
     """exp(x) / 0 and exp(x) / -0, one operand read by both: inf and -inf."""
     shape = [8192, 1024]
