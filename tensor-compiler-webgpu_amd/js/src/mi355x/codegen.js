@@ -413,7 +413,7 @@ function rowwiseKernel(b, output, opts) {
   // does not displace data that launch reads from the caches (tuning nto forces either way).
   const nt = (o.tuning || {}).nto === undefined ? o.streamOut === true : !!o.tuning.nto;
   const k = rowwiseText(b, [{ id: output, ptr: 'A.out', nt }], o, { args: 'TcmiArgs A', kind: 'row', at: (q) => `A.in[${q}]` });
-  k.merge = { body: b, output, rows: k.rows, held: k.held, tuning: o.tuning, streamed: o.lastReads || [], nt, sabotage: o.sabotage };
+  k.merge = { body: b, output, rows: k.rows, lanes: k.lanes, held: k.held, tuning: o.tuning, streamed: o.lastReads || [], nt, sabotage: o.sabotage };
   return k;
 }
 
@@ -613,7 +613,7 @@ ${indent(store, '    ')}
   const cap = (o.tuning && o.tuning.blocks) || 65536;
   const groups = Math.max(1, Math.min(Math.ceil(R / G), cap));
   return { name: k.name, source: k.source, params: Uint32Array.from(params), grid: [groups, 1, 1], block: [BLOCK, 1, 1], lds: 0, workspace: 0,
-    rows: [R, C], held: fills.length * E * W };
+    rows: [R, C], lanes: T, held: fills.length * E * W };
 }
 
 // ---- column reductions (sum / max over a non-last axis) --------------------------------

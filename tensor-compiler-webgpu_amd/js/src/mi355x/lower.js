@@ -1304,11 +1304,21 @@ function batchPlan(launches, aliases, bytesOf) {
     const outs = total(u.map((l) => l.node));
     const apart = outs + u.reduce((q, l) => q + total(reads(l)), 0);
     if (5 * (outs + total([].concat(...u.map(reads)))) > 4 * apart) return null;
-    // Rows that a whole workgroup reduces: only where the batch moves 128 MiB or more, half of the
-    // last-level cache, which below that serves the second read (logSoftmax's gradient over
-    // [16384, 4096], 1.3 GB: 203 us apart, 172 merged; LayerNorm's over [2176, 960], under 60 MB:
-    // 16.5 apart, 17.5 merged).
-    if (apart < 2 ** 27 && cg.wideRows(u[0].kernels[0])) return null;
+    // From 128 MiB (half of the last-level cache) rowwise members are bound by the bytes that a merge
+    // saves: LayerNorm's gradient over [8192, 960] 49.6 us apart, 41.2 merged. Below that:
+    if (apart < 2 ** 27) {
+      const k = u[0].kernels[0], blocks = k.grid[0], lanes = k.merge && k.merge.lanes;
+      // Few rows that a workgroup reduces run as one ragged batch, more of them as a dispatch each:
+      // softmax's gradient over [512, 2048] 4.1 us apart, 4.5 merged; [513, 2048] 6.9 / 4.6.
+      if (cg.wideRows(k) && blocks <= cg.RAGGED_MAX_BLOCKS) return null;
+      // A merged kernel reduces for one member after another, which a wavefront that holds one
+      // row only waits for; members side by side meet a row's second reader in the same XCD's L2 if
+      // their workgroups are a multiple of the 8 XCDs. Three members: LayerNorm's gradient over [2176, 960] 16.4 us
+      // apart, 17.4 merged, [4096, 768] 20.1 / 21.4, [6144, 512] 20.0 / 21.8; [3000, 512] (750
+      // workgroups) 17.3 / 15.4; two rows a wavefront [8192, 256] 15.1 / 14.7, [12288, 256] 19.6 /
+      // 20.6. Two members gain all the same: softmax's gradient over [6144, 512] 11.0 / 9.3.
+      if (lanes === 64 && u.length > 2 && blocks % 8 === 0) return null;
+    }
     return cg.mergedKernel(u.map((l) => ({ kernel: l.kernels[0], reads: reads(l) })));
   };
   // Launches of rows that a workgroup reduces are grouped only where they merge.

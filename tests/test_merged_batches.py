@@ -65,6 +65,18 @@ def test_wide_rows_that_do_not_merge_share_dispatches_as_other_launches_do(tool)
     assert [r["merged"] for r in res[:-1]] == [[]] * (len(res) - 1) and res[-1]["merged"][0]["count"] == 2
 
 
+def test_rowwise_members_merge_where_it_was_measured_faster(tool):
+    """Below 128 MiB: members whose wavefronts hold one row each, three or more of them over a multiple of 8 workgroups,
+    stay side by side; few wide rows stay a ragged batch; the others merge, as all do from 128 MiB."""
+    ln = [(2176, 960, 0), (4096, 768, 0), (8192, 256, 3), (3000, 512, 3), (8192, 960, 3), (512, 2048, 0), (513, 2048, 3)]
+    sm = [(6144, 512, 2), (512, 2048, 0), (513, 2048, 2), (1024, 4096, 2)]
+    g = tool("config-graphs", {"ln": [{"R": R, "C": C} for R, C, _ in ln], "c3": [{"fn": "softmax", "R": R, "C": C} for R, C, _ in sm]})
+    res = tool("batch-check", {"graphs": [dict(x["gradient"], name=f"{x.get('fn', 'layernorm')} {x['R']}x{x['C']}") for x in g["ln"] + g["c3"]]})
+    assert all(r["check"]["ok"] for r in res), [r for r in res if not r["check"]["ok"]]
+    rows = [[m["count"] for m in r["merged"] if m["kernel"].startswith("tcmi_grow")] for r in res]
+    assert rows == [[n] if n else [] for _, _, n in ln + sm], [(r["name"], x) for r, x in zip(res, rows)]
+
+
 def over_zeros():
     """exp(x) / 0 and exp(x) / -0, one operand read by both: inf and -inf."""
     shape = [8192, 1024]
