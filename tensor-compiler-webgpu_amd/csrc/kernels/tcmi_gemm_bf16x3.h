@@ -208,6 +208,7 @@ __device__ __forceinline__ void gemm_bf16x3(const Args& A, const float* __restri
                                             const uint32_t K, const uint32_t N, const uint32_t chunks, const uint32_t chunkK,
                                             const uint32_t zid, const uint32_t tx, const uint32_t ty) {
   static_assert(WM == 2, "gemm_f32_sum's wavefront rows");
+  static_assert(TN > 1, "a slice's splits stand beside every column of tiles but the last");
   constexpr int THREADS = 64 * WM * WN;
   constexpr int BM = WM * TM * 16, BN = WN * TN * 16;
   using SA = Bf16x3Stage<AV, false, BM, THREADS, AKC, KT>;

@@ -1143,7 +1143,7 @@ async function main() {
     case 'lower': {
       const g = Graph.fromJSON(req.graph);
       const target = req.fuse ? fuse(g, { keep: req.fuse.keep || [], recompute: !!req.fuse.recompute }).graph : g;
-      const l = lowerMI355X(target, req.perf ? { perf: true, keep: req.keep } : { sabotage: req.sabotage });
+      const l = lowerMI355X(target, req.perf ? { perf: true, keep: req.keep } : { sabotage: req.sabotage, tuning: req.tuning });
       out = { workspace: l.workspace, launches: l.launches.map((x) => Object.assign({}, x, { params: Array.from(x.params),
         kernels: x.kernels.map((k) => ({ name: k.name, grid: k.grid, block: k.block, lds: k.lds, source: req.sources ? k.source : undefined })) })) };
       break;

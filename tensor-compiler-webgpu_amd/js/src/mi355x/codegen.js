@@ -844,7 +844,9 @@ function gemmTiling(batch, M, N, K, tuning, peers) {
   // Unpadded products (above) take two groups up to 1024 tiles (the logits: 7.2 -> 6.7 us).
   const kw = t.kw || (T === 1 && chunks === 1 && blocks(1) <= 512 && K >= 256 ? (K >= 512 ? 4 : 2)
     : unpad && chunks === 1 && blocks(1) <= 1024 && K >= 256 ? 2 : 1);
-  const bf3 = t.bf3 === undefined && !t.tile && !t.waves && !t.kw && t.splitk === undefined && kw === 1 ? bf16x3Tiling(batch, M, N, K, P, chunks) : null;
+  // A tuning is of the fp32 kernel.
+  const tuned = ['tile', 'waves', 'kw', 'splitk', 'pad', 'bk', 'pf', 'prio', 'tm', 'tn'].some((x) => t[x] !== undefined);
+  const bf3 = !tuned && kw === 1 ? bf16x3Tiling(batch, M, N, K, P, chunks) : null;
   if (bf3) return bf3;
   const bk = t.bk || (kw > 1 ? 32 : wn === 4 ? 32 : T === 1 ? 64 : T === 2 ? 32 : 16);
   const pf = t.pf || 2;
@@ -852,7 +854,7 @@ function gemmTiling(batch, M, N, K, tuning, peers) {
   // Per-wavefront accumulator tiles along M (tm) and N (tn): T x T unless tuned.
   const tm = t.tm || T, tn = t.tn || T;
   const wide = batch * Math.ceil(M / (32 * tm)) * Math.ceil(N / (16 * wn * tn));
-  return { T, tm, tn, chunks, chunkK, bk, pf, wn, prio, kw, bf3: !!t.bf3, blocks: wide * chunks };
+  return { T, tm, tn, chunks, chunkK, bk, pf, wn, prio, kw, blocks: wide * chunks };
 }
 
 // The tiles of tcmi_gemm_bf16x3.h's kernel, and the relative time of one on a CU per output

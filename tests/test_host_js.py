@@ -392,6 +392,17 @@ def test_perf_lowering_keeps_the_split_of_config4_backward(tool):
             assert l["split"] == l["plainSplit"], (g["M"], g["K"], g["N"], l["node"])
 
 
+@pytest.mark.parametrize("tuning", [{"bk": 32}, {"pf": 1}, {"prio": False}, {"tm": 2}, {"tn": 2}, {"pad": False}, {"tile": 2}, {"splitk": 2}])
+def test_a_tuned_matmul_is_the_fp32_kernel_it_tunes(tool, tuning):
+    """A large product, which untuned takes the bf16 matrix cores."""
+    shape = [4096, 4096]
+    graph = {"nodes": [{"op": "input", "inputs": [], "attrs": {"name": n, "shape": shape}, "shape": shape} for n in "xw"]
+             + [{"op": "matmul", "inputs": [0, 1], "attrs": {}, "shape": shape}]}
+    kernel = [tool("lower", {"graph": graph, "sources": True, "tuning": t})["launches"][0]["kernels"][0]["source"] for t in (None, {"gemm": tuning})]
+    assert "gemm_bf16x3<" in kernel[0] and "gemm_f32<" not in kernel[0]
+    assert "gemm_f32<" in kernel[1] and "gemm_bf16x3<" not in kernel[1]
+
+
 def test_row_fold_takes_in_a_producer_only_with_a_full_size_body(tool):
     """A row reduction's elementwise producer joins the reduction's rowwise launch only when
     every value of its body is full size (besides its operands, constants and their
