@@ -7,7 +7,8 @@ quoted on first: fused elementwise chains — 8 seeded programs of 8–16 ops ov
 fp32 [8192, 1024] with a [1024] row-vector broadcast, each run forward and as
 its autodiff gradient graph — in algorithmic HBM GB/s (every unique operand of
 a launch read once at its own size, plus its output: the reference's byte
-count, src/fusion/workloads.js:171-172) of the launches this backend runs. A
+count, src/fusion/workloads.js:171-172) of the launches this backend runs, an
+operand that one kernel loads for several merged launches counted once. A
 step is one run of every fused program; K steps are timed between a sync and
 hipEvents on both sides, with the inputs already in HBM. The perf lowering
 forms some values inside the launches that read them, so it moves fewer bytes

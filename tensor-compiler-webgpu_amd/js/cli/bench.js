@@ -32,7 +32,7 @@
 
 const { size } = require('../src/ir/shapes');
 const { fuse } = require('../src/fusion/fuse');
-const { lowerMI355X } = require('../src/mi355x/lower');
+const { lowerMI355X, movedBytes } = require('../src/mi355x/lower');
 const { HipRunner, Concurrent } = require('../src/mi355x/runner');
 const { HipBench, summarize, verdict, median } = require('../src/mi355x/bench');
 const { chainWorkload, chainInputs } = require('../src/builders/chains');
@@ -62,7 +62,9 @@ function prepared(runner, graph, lowered, inputs, opts) {
  * proportion to their work (flops where every member has them, algorithmic bytes where
  * none has: evenly among identical members; members whose bodies differ may differ in
  * size), so a member costs what it costs inside its batch, not what it would cost by
- * itself. A ragged batch's members are timed each alone.
+ * itself. A ragged batch's members are timed each alone. `moved`: the
+ * member's share of what its dispatch moves, less than its own `bytes` where a merged batch loads
+ * an operand once for several.
  */
 function timeLaunches(runner, bench, program, reps) {
   const out = [];
@@ -81,9 +83,10 @@ function timeLaunches(runner, bench, program, reps) {
     const byFlops = members.every((l) => l.flops > 0);
     const work = members.map((l) => (byFlops ? l.flops : l.bytes || 0));
     const total = work.reduce((s, w) => s + w, 0);
+    const loaded = b && b.merged ? b.bytes / members.reduce((s, l) => s + l.bytes, 0) : 1;
     members.forEach((l, k) => {
       const share = total > 0 ? work[k] / total : 1 / n;
-      out.push({ node: l.node, kind: l.kind, pattern: l.pattern || null, code: l.code, bytes: l.bytes, flops: l.flops,
+      out.push({ node: l.node, kind: l.kind, pattern: l.pattern || null, code: l.code, bytes: l.bytes, moved: l.bytes * loaded, flops: l.flops,
         us: r.stats.one.median * share, minUs: r.stats.one.min * share, maxUs: r.stats.one.max * share, rowFolds: l.rowFolds || null, absorbed: l.absorbed || null,
         formed: l.formed || null, batched: n > 1 ? n : undefined, joint: b && b.joint ? true : undefined });
     });
@@ -200,7 +203,7 @@ function measureGraph(runner, bench, name, graph, keep, inputs, opts) {
     total += a.length;
     for (let i = 0; i < a.length; i++) if (Object.is(a[i], b[i])) same++;
   }
-  const bytesF = lf.launches.reduce((s, l) => s + l.bytes, 0);
+  const bytesF = movedBytes(lf);
   const bytesU = lu.launches.reduce((s, l) => s + l.bytes, 0);
   // The fusion contract's count of the same program: one launch per fused node (the
   // reference's own accounting of a fused program, workloads.js:155-175).
@@ -229,8 +232,8 @@ function measureGraph(runner, bench, name, graph, keep, inputs, opts) {
 function dominant(launches) {
   const by = new Map();
   for (const l of launches) {
-    const e = by.get(l.code) || { code: l.code, kind: l.kind, pattern: l.pattern, count: 0, us: 0, bytes: 0, flops: 0 };
-    e.count++; e.us += l.us; e.bytes += l.bytes; e.flops += l.flops || 0;
+    const e = by.get(l.code) || { code: l.code, kind: l.kind, pattern: l.pattern, count: 0, us: 0, bytes: 0, moved: 0, flops: 0 };
+    e.count++; e.us += l.us; e.bytes += l.bytes; e.moved += l.moved === undefined ? l.bytes : l.moved; e.flops += l.flops || 0;
     by.set(l.code, e);
   }
   let best = null;
@@ -238,7 +241,7 @@ function dominant(launches) {
   for (const e of by.values()) if (!best || weight(e) > weight(best)) best = e;
   if (!best) return null;
   const avgUs = best.us / best.count, bytes = best.bytes / best.count;
-  return Object.assign(best, { avgUs, bytesPerLaunch: bytes, gbs: bytes / (avgUs * 1e3),
+  return Object.assign(best, { avgUs, bytesPerLaunch: bytes, gbs: best.moved / (best.us * 1e3),
     tflops: best.flops ? best.flops / best.count / (avgUs * 1e6) : null });
 }
 
@@ -339,7 +342,7 @@ function c2(runner, bench, opts) {
         const lf = lowerMI355X(f.graph, { perf: true, keep: v.keep.map((id) => f.index.get(id)) });
         runner.functions(lf);
         programs.push(prepared(runner, f.graph, lf, inputs, arena ? { arena: { keep: v.keep.map((id) => f.index.get(id)) } } : undefined));
-        results.push({ name: `c2-p${s}-${kind}`, bytes: { fused: lf.launches.reduce((q, l) => q + l.bytes, 0),
+        results.push({ name: `c2-p${s}-${kind}`, bytes: { fused: movedBytes(lf),
           contract: lowerMI355X(f.graph).launches.reduce((q, l) => q + l.bytes, 0) }, launchF: [],
           launches: launchRecords(lf) });
         continue;
@@ -445,16 +448,17 @@ function runOnly(runner, name, graph, keep, inputs, fuseOptions) {
 
 /**
  * Every launch of a lowering with its kernel names, algorithmic bytes and flops (for
- * profile summaries); each batched launch as one more record, its members' work summed.
+ * profile summaries); each batched launch as one more record, its members' work summed (bytes: a merged
+ * batch's operands once each).
  */
 function launchRecords(lowered) {
   const recs = lowered.launches.map((l) => ({ node: l.node, kind: l.kind, pattern: l.pattern || null,
     kernels: l.kernels.map((k) => k.name), bytes: l.bytes, flops: l.flops || 0 }));
   for (const b of lowered.batches || []) {
     const ms = lowered.launches.slice(b.start, b.start + b.count);
-    const kind = b.ragged ? `ragged x${b.count} (${Array.from(new Set(ms.map((l) => l.kind))).join(', ')})` : `batched ${ms[0].kind} x${b.count}`;
+    const kind = b.ragged ? `ragged x${b.count} (${Array.from(new Set(ms.map((l) => l.kind))).join(', ')})` : `${b.merged ? 'merged' : 'batched'} ${ms[0].kind} x${b.count}`;
     recs.push({ node: ms[0].node, kind, pattern: ms[0].pattern || null, kernels: b.kernels.map((k) => k.name),
-      bytes: ms.reduce((q, l) => q + l.bytes, 0), flops: ms.reduce((q, l) => q + (l.flops || 0), 0), members: ms.map((l) => l.node) });
+      bytes: b.merged ? b.bytes : ms.reduce((q, l) => q + l.bytes, 0), flops: ms.reduce((q, l) => q + (l.flops || 0), 0), members: ms.map((l) => l.node) });
   }
   return recs;
 }
@@ -657,7 +661,7 @@ function trainStep(runner, bench, name, req, opts) {
   const byKind = {};
   for (const l of launches) {
     const e = byKind[l.kind] || (byKind[l.kind] = { launches: 0, us: 0, bytes: 0, flops: 0 });
-    e.launches++; e.us += l.us; e.bytes += l.bytes; e.flops += l.flops || 0;
+    e.launches++; e.us += l.us; e.bytes += l.moved; e.flops += l.flops || 0;
   }
   for (const k of Object.keys(byKind)) {
     const e = byKind[k];
@@ -774,7 +778,8 @@ function sweep(runner, bench, opts) {
       runner.functions(lowered);
       const launches = lowered.launches.filter((l) => !only || only(l));
       variants[v] = prepared(runner, graph, lowered, m.inputs, only ? { only } : undefined);
-      info[v] = { launches: launches.length, bytes: launches.reduce((q, l) => q + l.bytes, 0), flops: launches.reduce((q, l) => q + (l.flops || 0), 0) };
+      info[v] = { launches: launches.length, bytes: only ? launches.reduce((q, l) => q + l.bytes, 0) : movedBytes(lowered),
+        flops: launches.reduce((q, l) => q + (l.flops || 0), 0) };
     }
     const t = bench.time(variants, { reps: opts.reps || 16 });
     const row = { id: w.id, family: w.family, params: w.params, gate: g, timed: true, k: t.k, variants: {} };

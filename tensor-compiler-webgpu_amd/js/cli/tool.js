@@ -37,7 +37,7 @@ const { Graph } = require('../src/ir/graph');
 const { size } = require('../src/ir/shapes');
 const { grad } = require('../src/autodiff');
 const { fuse, fusionSummary } = require('../src/fusion/fuse');
-const { lowerMI355X, kernelSources } = require('../src/mi355x/lower');
+const { lowerMI355X, kernelSources, movedBytes } = require('../src/mi355x/lower');
 const { builderCases } = require('../src/testing/cases');
 const { fusedDirectCases } = require('../src/builders/direct_cases');
 const tf = require('../src/builders/transformer');
@@ -1429,7 +1429,8 @@ async function main() {
       const one = (name, graph, keep, absorb = true) => {
         const plain = lowerMI355X(graph, { perf: true, keep, batch: false, absorb });
         const batched = lowerMI355X(graph, { perf: true, keep, absorb });
-        const res = { name, launches: batched.launches.length, check: checkBatches(plain, batched),
+        const res = { name, launches: batched.launches.length, check: checkBatches(plain, batched), bytes: movedBytes(batched),
+          apart: batched.launches.reduce((q, l) => q + l.bytes, 0),
           merged: (batched.batches || []).filter((b) => b.merged).map((b) => ({ count: b.count, kind: batched.launches[b.start].kind, kernel: b.kernels[0].name })) };
         if (req.plant) {
           for (const kind of ['dependent', 'early', 'grid', 'body']) {

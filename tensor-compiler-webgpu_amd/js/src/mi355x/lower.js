@@ -1281,8 +1281,8 @@ function lowerOnce(graph, opts, noAbsorb, noForm) {
  * runs its launches' kernels over all members in turn (all first kernels, then
  * all second kernels), member k with the workspace slice
  * [k·wsStride, (k + 1)·wsStride). Returns { launches (the new order), batches:
- * [{ start, count, kernels, wsStride, ragged?, joint? }] } with each batch's members at
- * launches[start .. start + count).
+ * [{ start, count, kernels, wsStride, ragged?, joint?, merged?, bytes? }] } with each batch's members at
+ * launches[start .. start + count); bytes: a merged batch's, its members' operands once each.
  */
 function batchPlan(launches, aliases, bytesOf) {
   const owner = (id) => (aliases.has(id) ? aliases.get(id) : id);
@@ -1302,8 +1302,8 @@ function batchPlan(launches, aliases, bytesOf) {
     const total = (ids) => Array.from(new Set(ids)).reduce((q, id) => q + bytesOf(id), 0);
     const reads = (l) => l.inputs.map(owner);
     const outs = total(u.map((l) => l.node));
-    const apart = outs + u.reduce((q, l) => q + total(reads(l)), 0);
-    if (5 * (outs + total([].concat(...u.map(reads)))) > 4 * apart) return null;
+    const apart = outs + u.reduce((q, l) => q + total(reads(l)), 0), bytes = outs + total([].concat(...u.map(reads)));
+    if (5 * bytes > 4 * apart) return null;
     // From 128 MiB (half of the last-level cache) rowwise members are bound by the bytes that a merge
     // saves: LayerNorm's gradient over [8192, 960] 49.6 us apart, 41.2 merged. Below that:
     if (apart < 2 ** 27) {
@@ -1319,7 +1319,8 @@ function batchPlan(launches, aliases, bytesOf) {
       // 20.6. Two members gain all the same: softmax's gradient over [6144, 512] 11.0 / 9.3.
       if (lanes === 64 && u.length > 2 && blocks % 8 === 0) return null;
     }
-    return cg.mergedKernel(u.map((l) => ({ kernel: l.kernels[0], reads: reads(l) })));
+    const kernel = cg.mergedKernel(u.map((l) => ({ kernel: l.kernels[0], reads: reads(l) })));
+    return kernel && { kernel, bytes };
   };
   // Launches of rows that a workgroup reduces are grouped only where they merge.
   const wide = (l) => (l.kernels.length === 1 && cg.wideRows(l.kernels[0]) ? cg.mergeFamily(l.kernels[0]) : null);
@@ -1453,7 +1454,7 @@ function batchPlan(launches, aliases, bytesOf) {
     }
     const one = u.length > 1 ? merged(u) : null;
     if (one) {
-      batches.push({ start: order.length, count: u.length, kernels: [one], wsStride: 0, merged: true });
+      batches.push({ start: order.length, count: u.length, kernels: [one.kernel], wsStride: 0, merged: true, bytes: one.bytes });
     } else if (u.length > 1 && u.ragged) {
       batches.push({ start: order.length, count: u.length, kernels: [cg.raggedKernel(u.map((m) => m.kernels[0]))], wsStride: 0, ragged: true });
     } else if (u.length > 1) {
@@ -1466,6 +1467,18 @@ function batchPlan(launches, aliases, bytesOf) {
   return { launches: order, batches };
 }
 
+/**
+ * Algorithmic bytes of a lowering as it runs: every launch's unique operands and output once, and
+ * an operand that several members of a merged batch read, which their kernel loads once, once.
+ */
+function movedBytes(lowered) {
+  let bytes = lowered.launches.reduce((q, l) => q + l.bytes, 0);
+  for (const b of lowered.batches || []) {
+    if (b.merged) bytes += b.bytes - lowered.launches.slice(b.start, b.start + b.count).reduce((q, l) => q + l.bytes, 0);
+  }
+  return bytes;
+}
+
 /** Every distinct kernel source of a launch list (its batched kernels included), in first-use order. */
 function kernelSources(lowered) {
   const seen = new Map();
@@ -1474,4 +1487,4 @@ function kernelSources(lowered) {
   return seen;
 }
 
-module.exports = { lowerMI355X, kernelSources, batchPlan, lowerNode, oneOpBody, algorithmicBytes, chainMap };
+module.exports = { lowerMI355X, kernelSources, batchPlan, lowerNode, oneOpBody, algorithmicBytes, movedBytes, chainMap };

@@ -77,6 +77,23 @@ def test_rowwise_members_merge_where_it_was_measured_faster(tool):
     assert rows == [[n] if n else [] for _, _, n in ln + sm], [(r["name"], x) for r, x in zip(res, rows)]
 
 
+def test_merged_batches_count_an_operand_once(tool):
+    """The bytes of a lowering as it runs (the benchmark's step_bytes): config 2's 16 programs, of which merged batches load
+    shared operands once, and the logSoftmax gradient, which reads x and dy and writes y and dx."""
+    g = tool("config-graphs", {"c2": [{"seed": s, "R": 8192, "C": 1024} for s in range(8)], "c3": [{"fn": "logSoftmax", "R": 16384, "C": 4096}]})
+    res = tool("batch-check", {"graphs": [dict(x[k], name=f"chain-{x['seed']}-{k}") for x in g["c2"] for k in ("forward", "gradient")]
+                               + [dict(g["c3"][0]["gradient"], name="rows")]})
+    assert res[-1]["bytes"] == 4 * 4 * 16384 * 4096
+    tensor = 4 * 8192 * 1024
+    merged = [r for r in res[:-1] if r["merged"]]
+    # What one by one launches of the same lowering read and write, as the records of the launches add up to.
+    apart = {r["name"]: r["apart"] for r in res}
+    assert merged and all(apart[r["name"]] - r["bytes"] >= tensor for r in merged)
+    assert all(apart[r["name"]] == r["bytes"] for r in res[:-1] if not r["merged"])
+    assert apart["chain-0-gradient"] - res[1]["bytes"] == 8 * tensor + 4 * 1024    # and the row vector once
+    assert sum(r["bytes"] for r in res[:-1]) == 2449633280
+
+
 def over_zeros():
     """exp(x) / 0 and exp(x) / -0, one operand read by both: inf and -inf."""
     shape = [8192, 1024]
