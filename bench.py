@@ -44,6 +44,8 @@ sys.path.insert(0, str(PKG))
 METRIC = "fused-kernel HBM GB/s + matmul TFLOP/s (% roofline); transformer train steps/sec"
 HBM_PEAK = 8000.0
 MFMA_FP32_PEAK = 157.3
+# An fp32 product in bf16 parts is six bf16 ones, at a dense peak of 2500 TFLOP/s.
+MFMA_BF16_PARTS_PEAK = 2500.0 / 6
 
 
 def cpu_model() -> str:
@@ -350,8 +352,9 @@ def compose(full: dict) -> dict:
             t = (r["tflops"] or {}).get("fused")
             e = shapes.setdefault(shape, {})
             e[f"{act}_{'fwd' if kind == 'forward' else 'bwd'}_TFLOPs"] = _r(t)
-        for shape, e in shapes.items():
-            e["frac_fwd"] = _r(max(e.get("relu_fwd_TFLOPs") or 0, e.get("tanh_fwd_TFLOPs") or 0) / MFMA_FP32_PEAK)
+            if kind == "forward":
+                e["frac_fwd"] = max(e.get("frac_fwd", 0), _r((t or 0) / (MFMA_BF16_PARTS_PEAK if r.get("bf16Parts") else MFMA_FP32_PEAK)))
+                e["frac_of"] = "bf16 MFMA peak / 6" if r.get("bf16Parts") else "fp32 MFMA peak"
         extra["c4"] = shapes
         extra["c4_groups"] = _groups(c4.get("groups"))
     for key in ("c1", "c5"):

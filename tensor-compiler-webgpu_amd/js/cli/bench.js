@@ -217,6 +217,8 @@ function measureGraph(runner, bench, name, graph, keep, inputs, opts) {
     gbs: { fused: bytesF / (t.stats.fused.median * 1e3), unfused: bytesU / (t.stats.unfused.median * 1e3) },
     tflops: flops ? { fused: flops / (t.stats.fused.median * 1e6), unfused: flops / (t.stats.unfused.median * 1e6) } : null,
     bitwiseSameOutputs: { same, total }, groups, launchF, launchU,
+    // Whether its products run on the bf16 matrix cores, six times the flops each.
+    bf16Parts: lf.launches.some((l) => l.kernels[0].source.includes('gemm_bf16x3<')),
   };
   if (o.keepPrograms) res.programs = { pf, pu };
   else { pf.destroy(); pu.destroy(); }

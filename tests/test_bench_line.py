@@ -71,6 +71,18 @@ def test_every_config_is_carried_compactly(line):
     assert len(json.dumps(r, separators=(",", ":"))) < 6000
 
 
+def test_a_products_share_is_of_the_matrix_cores_it_runs_on():
+    """A forward product of 220 TFLOP/s: above the fp32 matrix cores' peak, half of the bf16 ones' in six parts."""
+    import bench
+    doc = json.loads((ROOT / "tests" / "golden" / "bench_document.json").read_text())
+    r = next(x for x in doc["configs"]["c4"]["results"] if x["name"].endswith("-relu-forward"))
+    doc["configs"]["c4"]["results"] = [dict(r, name=f"c4-{n}-relu-forward", tflops=dict(r["tflops"], fused=t), bf16Parts=parts)
+                                       for n, t, parts in (("1x1x1", 220.0, True), ("2x2x2", 51.0, False))]
+    c4 = bench.compose(doc)["extra"]["c4"]
+    assert c4["1x1x1"]["frac_fwd"] == pytest.approx(220 * 6 / 2500, abs=1e-3) and c4["1x1x1"]["frac_of"].startswith("bf16")
+    assert c4["2x2x2"]["frac_fwd"] == pytest.approx(51 / 157.3, abs=1e-3) and c4["2x2x2"]["frac_of"].startswith("fp32")
+
+
 def test_a_cold_figure_above_the_read_ceiling_is_marked():
     """compose() marks a roofline figure above the pure-read ceiling of the same run as
     cache-assisted instead of reporting it as an HBM figure (planted: the document's cold
