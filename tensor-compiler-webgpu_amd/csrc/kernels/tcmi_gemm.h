@@ -115,9 +115,9 @@ __device__ __forceinline__ float4 vop(float4 x) {
 
 // A per-element (MODE_S) operand one of whose indices is contiguous all the same, its rows of a
 // length or at an offset that is no multiple of 4: V::RUN 1 names the column, 2 the row. It is
-// staged as MODE_C or MODE_R, by 128-bit loads of 4-byte alignment, single ones where a
-// group of 4 crosses the end of the run. (777 x 1000 x 515, both operands such: 20.9 us
-// against 34.2 with one load per element; 1000 x 777 x 515 20.3 against 28.1.)
+// staged as MODE_C or MODE_R, by 128-bit loads of 4-byte alignment. (777 x 1000 x 515, both operands such: 20.9 us
+// against 34.2 with one load per element; 96 x 1088 x 378 10.4 against 11.5, where single loads
+// for the groups that cross the end of the run, behind a branch, took 12.5.)
 template <class V>
 __device__ constexpr auto view_run(int) -> decltype(V::RUN, int()) { return V::RUN; }
 template <class V>
@@ -127,13 +127,18 @@ __device__ constexpr int staged_mode() {
   return MODE != MODE_S ? MODE : view_run<V>(0) == 1 ? static_cast<int>(MODE_C) : view_run<V>(0) == 2 ? static_cast<int>(MODE_R) : static_cast<int>(MODE_S);
 }
 typedef float run4 __attribute__((ext_vector_type(4), aligned(4)));
-// Four elements of a run at p, of which `left` (1 or more) are inside the operand; 0 past them.
-__device__ __forceinline__ float4 load_run4(const float* p, uint32_t left) {
-  if (left >= 4u) {
-    const run4 r = *reinterpret_cast<const run4*>(p);
-    return make_float4(r[0], r[1], r[2], r[3]);
-  }
-  return make_float4(p[0], left > 1u ? p[1] : 0.f, left > 2u ? p[2] : 0.f, 0.f);
+// Elements by which the group of 4 at `at` (inside its run, of 4 or more) passes the run's end. The group is
+// loaded so much early, inside the run, and moved into place as it is stored to LDS (run_shift, the rest 0):
+// no branch, so the load waits for nothing.
+__device__ __forceinline__ uint32_t run_over(uint32_t at, uint32_t end) { return at < end && at + 4u > end ? at + 4u - end : 0u; }
+__device__ __forceinline__ float4 load_run4(const float* p, uint32_t over) {
+  const run4 r = *reinterpret_cast<const run4*>(p - over);
+  return make_float4(r[0], r[1], r[2], r[3]);
+}
+__device__ __forceinline__ float4 run_shift(float4 x, uint32_t over) {
+  if (over & 1u) x = make_float4(x.y, x.z, x.w, 0.f);
+  if (over & 2u) x = make_float4(x.z, x.w, 0.f, 0.f);
+  return x;
 }
 
 // A workgroup's (x, y, z) place in its launch's grid.
@@ -221,7 +226,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const uint32_t row = t / (BK / 4), kk = (t % (BK / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
         if (t < BM * BK / 4 && m0 + row < M && k0 + kk < kend) {
-          if constexpr (view_run<AV>(0) != 0) x = load_run4(Ab + vrow<AV>(m0 + row) + vcol<AV>(k0 + kk), kend - (k0 + kk));
+          if constexpr (view_run<AV>(0) != 0) x = load_run4(Ab + vrow<AV>(m0 + row) + vcol<AV>(k0 + kk), run_over(k0 + kk, kend));
           else x = *reinterpret_cast<const float4*>(Ab + vrow<AV>(m0 + row) + vcol<AV>(k0 + kk));
         }
         ra[v] = x;
@@ -233,7 +238,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const uint32_t kk = t / (BM / 4), row = (t % (BM / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
         if (t < BM * BK / 4 && m0 + row < M && k0 + kk < kend) {
-          if constexpr (view_run<AV>(0) != 0) x = load_run4(Ab + vcol<AV>(k0 + kk) + vrow<AV>(m0 + row), M - (m0 + row));
+          if constexpr (view_run<AV>(0) != 0) x = load_run4(Ab + vcol<AV>(k0 + kk) + vrow<AV>(m0 + row), run_over(m0 + row, M));
           else x = *reinterpret_cast<const float4*>(Ab + vcol<AV>(k0 + kk) + vrow<AV>(m0 + row));
         }
         ra[v] = x;
@@ -255,7 +260,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const uint32_t kk = t / (BN / 4), c = (t % (BN / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
         if (t < BK * BN / 4 && k0 + kk < kend && n0 + c < N) {
-          if constexpr (view_run<BV>(0) != 0) x = load_run4(Bb + vrow<BV>(k0 + kk) + vcol<BV>(n0 + c), N - (n0 + c));
+          if constexpr (view_run<BV>(0) != 0) x = load_run4(Bb + vrow<BV>(k0 + kk) + vcol<BV>(n0 + c), run_over(n0 + c, N));
           else x = *reinterpret_cast<const float4*>(Bb + vrow<BV>(k0 + kk) + vcol<BV>(n0 + c));
         }
         rb[v] = x;
@@ -267,7 +272,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const uint32_t c = t / (BK / 4), kk = (t % (BK / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
         if (t < BK * BN / 4 && k0 + kk < kend && n0 + c < N) {
-          if constexpr (view_run<BV>(0) != 0) x = load_run4(Bb + vcol<BV>(n0 + c) + vrow<BV>(k0 + kk), kend - (k0 + kk));
+          if constexpr (view_run<BV>(0) != 0) x = load_run4(Bb + vcol<BV>(n0 + c) + vrow<BV>(k0 + kk), run_over(k0 + kk, kend));
           else x = *reinterpret_cast<const float4*>(Bb + vcol<BV>(n0 + c) + vrow<BV>(k0 + kk));
         }
         rb[v] = x;
@@ -284,7 +289,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
     }
   };
 
-  auto store_slice = [&](const Stage& S, int buf) {
+  auto store_slice = [&](const Stage& S, int buf, uint32_t k0) {
     const float4* ra = S.ra;
     const float4* rb = S.rb;
     const float* sa = S.sa;
@@ -295,7 +300,9 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const int t = tid + v * THREADS;
         if (t < BM * BK / 4) {
           const int row = t / (BK / 4), kk = (t % (BK / 4)) * 4;
-          *reinterpret_cast<float4*>(&As[buf][row * AS + kk]) = vop<AV>(ra[v]);
+          float4 x = ra[v];
+          if (view_run<AV>(0) != 0 && k0 + BK > kend) x = run_shift(x, run_over(k0 + kk, kend));
+          *reinterpret_cast<float4*>(&As[buf][row * AS + kk]) = vop<AV>(x);
         }
       }
     } else if (AM == MODE_R) {
@@ -304,7 +311,9 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const int t = tid + v * THREADS;
         if (t < BM * BK / 4) {
           const int kk = t / (BM / 4), row = (t % (BM / 4)) * 4;
-          *reinterpret_cast<float4*>(&As[buf][kk * AS + row]) = vop<AV>(ra[v]);
+          float4 x = ra[v];
+          if (view_run<AV>(0) != 0 && m0 + BM > M) x = run_shift(x, run_over(m0 + row, M));
+          *reinterpret_cast<float4*>(&As[buf][kk * AS + row]) = vop<AV>(x);
         }
       }
     } else {
@@ -320,7 +329,9 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const int t = tid + v * THREADS;
         if (t < BK * BN / 4) {
           const int kk = t / (BN / 4), c = (t % (BN / 4)) * 4;
-          *reinterpret_cast<float4*>(&Bs[buf][kk * BS + c]) = vop<BV>(rb[v]);
+          float4 x = rb[v];
+          if (view_run<BV>(0) != 0 && n0 + BN > N) x = run_shift(x, run_over(n0 + c, N));
+          *reinterpret_cast<float4*>(&Bs[buf][kk * BS + c]) = vop<BV>(x);
         }
       }
     } else if (BMD == MODE_R) {
@@ -329,7 +340,9 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const int t = tid + v * THREADS;
         if (t < BK * BN / 4) {
           const int c = t / (BK / 4), kk = (t % (BK / 4)) * 4;
-          *reinterpret_cast<float4*>(&Bs[buf][c * BS + kk]) = vop<BV>(rb[v]);
+          float4 x = rb[v];
+          if (view_run<BV>(0) != 0 && k0 + BK > kend) x = run_shift(x, run_over(k0 + kk, kend));
+          *reinterpret_cast<float4*>(&Bs[buf][c * BS + kk]) = vop<BV>(x);
         }
       }
     } else {
@@ -392,7 +405,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
   };
 
   load_slice(st0, kbeg);
-  store_slice(st0, 0);
+  store_slice(st0, 0, kbeg);
   if (PF == 2 && slices > 1) load_slice(st1, kbeg + BK);
   __syncthreads();
   if (PF == 1) {
@@ -400,7 +413,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
       const int cur = ks & 1;
       if (ks + 1 < slices) load_slice(st0, kbeg + (ks + 1) * BK);
       compute(cur);
-      if (ks + 1 < slices) store_slice(st0, cur ^ 1);
+      if (ks + 1 < slices) store_slice(st0, cur ^ 1, kbeg + (ks + 1) * BK);
       __syncthreads();
     }
   } else {
@@ -409,12 +422,12 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
     for (uint32_t ks = 0; ks < slices; ks += 2) {
       if (ks + 2 < slices) load_slice(st0, kbeg + (ks + 2) * BK);
       compute(0);
-      if (ks + 1 < slices) store_slice(st1, 1);
+      if (ks + 1 < slices) store_slice(st1, 1, kbeg + (ks + 1) * BK);
       __syncthreads();
       if (ks + 1 >= slices) break;
       if (ks + 3 < slices) load_slice(st1, kbeg + (ks + 3) * BK);
       compute(1);
-      if (ks + 2 < slices) store_slice(st0, 0);
+      if (ks + 2 < slices) store_slice(st0, 0, kbeg + (ks + 2) * BK);
       __syncthreads();
     }
   }

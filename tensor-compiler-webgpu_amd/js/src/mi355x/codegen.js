@@ -983,7 +983,8 @@ function operandView(name, view, batchDims, R, C) {
   if (v.sc === 1 && C % 4 === 0 && others4(v.sr)) mode = 0;
   else if (v.sr === 1 && R % 4 === 0 && others4(v.sc)) mode = 1;
   // A per-element operand whose elements still lie in runs (tcmi_gemm.h view_run). Runs shorter than
-  // two tiles are mostly their ends: config 1's 128 x 128 x 10 product 4.1 us per element, 4.7 as runs.
+  // two tiles are mostly their ends: config 1's 128 x 128 x 10 product 4.3 us per element, 4.8 as runs,
+  // 1000 x 30 x 50 3.9 / 4.8.
   const run = mode !== 2 ? 0 : v.sc === 1 && C >= 64 ? 1 : v.sr === 1 && R >= 64 ? 2 : 0;
   const text = `struct ${name} {
   static constexpr size_t SR = ${v.sr}, SC = ${v.sc};${loadOp(v)}${run ? `\n  static constexpr int RUN = ${run};` : ''}

@@ -9,7 +9,7 @@ import pytest
 
 CHAINS = [(0, 8192, 1024), (3, 8192, 1024), (11, 4097, 515), (13, 4097, 515), (0, 4097, 515), (13, 2049, 1024), (3, 64, 1024)]
 ROWS = [("softmax", 16384, 4096), ("logSoftmax", 16384, 4096), ("softmax", 8191, 258), ("logSoftmax", 4099, 2049), ("softmax", 8193, 61),
-        ("softmax", 64, 258)]
+        ("softmax", 64, 258), ("softmax", 300, 3000), ("logSoftmax", 513, 2048)]
 
 
 def graphs(tool):
