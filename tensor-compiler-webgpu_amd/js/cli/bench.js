@@ -454,12 +454,13 @@ function runOnly(runner, name, graph, keep, inputs, fuseOptions) {
  * batch's operands once each).
  */
 function launchRecords(lowered) {
+  const bf16Parts = (ks) => ks.some((k) => k.source.includes('gemm_bf16x3<'));
   const recs = lowered.launches.map((l) => ({ node: l.node, kind: l.kind, pattern: l.pattern || null,
-    kernels: l.kernels.map((k) => k.name), bytes: l.bytes, flops: l.flops || 0 }));
+    kernels: l.kernels.map((k) => k.name), bytes: l.bytes, flops: l.flops || 0, bf16Parts: bf16Parts(l.kernels) }));
   for (const b of lowered.batches || []) {
     const ms = lowered.launches.slice(b.start, b.start + b.count);
     const kind = b.ragged ? `ragged x${b.count} (${Array.from(new Set(ms.map((l) => l.kind))).join(', ')})` : `${b.merged ? 'merged' : 'batched'} ${ms[0].kind} x${b.count}`;
-    recs.push({ node: ms[0].node, kind, pattern: ms[0].pattern || null, kernels: b.kernels.map((k) => k.name),
+    recs.push({ node: ms[0].node, kind, pattern: ms[0].pattern || null, kernels: b.kernels.map((k) => k.name), bf16Parts: bf16Parts(b.kernels),
       bytes: b.merged ? b.bytes : ms.reduce((q, l) => q + l.bytes, 0), flops: ms.reduce((q, l) => q + (l.flops || 0), 0), members: ms.map((l) => l.node) });
   }
   return recs;

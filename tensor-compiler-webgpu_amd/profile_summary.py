@@ -8,7 +8,7 @@
 Inputs are what `node js/cli/bench.js --step-only` prints (every launch of every
 program with its kernel names, algorithmic bytes and flops) and the CSV files that
 `rocprofv3 --kernel-trace --stats -f csv` and `rocprofv3 --pmc FETCH_SIZE` /
-`--pmc WRITE_SIZE` (and optionally `--pmc MfmaUtil MfmaFlopsF32 LDSBankConflict`)
+`--pmc WRITE_SIZE` (and optionally `--pmc MfmaUtil MfmaFlopsF32 MfmaFlopsBF16 LDSBankConflict`)
 write for the same command. The counter passes are calibrated on the bench's 1 GiB
 copy kernel (k_copy16, run in the same process by `--configs ceiling,...`): the
 factor that turns its FETCH_SIZE and WRITE_SIZE (KiB per dispatch) into 1 GiB is
@@ -29,6 +29,7 @@ import pathlib
 
 HBM_PEAK_GBS = 8000.0
 MFMA_FP32_PEAK_TFLOPS = 157.3
+MFMA_BF16_PARTS_PEAK_TFLOPS = 2500.0 / 6     # an fp32 product in bf16 parts is six bf16 ones
 GIB_KIB = 1024 * 1024
 
 
@@ -50,7 +51,7 @@ def launch_info(bench: dict, configs) -> dict:
                     # A launch's algorithmic work belongs to its first kernel; the others
                     # (split-K chunk sums, column sums' second pass) carry none of their own.
                     e = info.setdefault(k, {"kind": l["kind"] if i == 0 else f"{l['kind']} (second pass)",
-                                            "pattern": l["pattern"], "programs": set(),
+                                            "pattern": l["pattern"], "programs": set(), "parts": bool(l.get("bf16Parts")),
                                             "bytes": l["bytes"] if i == 0 else 0, "flops": l["flops"] if i == 0 else 0})
                     e["programs"].add(r["name"])
     return info
@@ -83,7 +84,7 @@ def summarize(a) -> str:
            f"{GIB_KIB / wf:.0f} KiB per dispatch for 1 GiB each way: FETCH_SIZE x {ff:.4f}, WRITE_SIZE x {wf:.4f}.", ""]
     head = "| kernel | kind | programs | calls | avg us | algorithmic | achieved | of peak | HBM traffic / launch | traffic / algorithmic bytes |"
     if mfma:
-        head += " MfmaUtil | MfmaFlopsF32 / flops | LDS conflict |"
+        head += " MfmaUtil | MfmaFlopsF32 / flops | MfmaFlopsBF16 / flops | LDS conflict |"
     out += [head, "|" + "---|" * (head.count("|") - 1)]
     for k, e, calls, avg, t in rows:
         progs = ", ".join(sorted(e["programs"]))
@@ -93,7 +94,7 @@ def summarize(a) -> str:
         if e["flops"]:
             alg = f"{e['flops'] / 1e9:.2f} GFLOP"
             rate = e["flops"] / (avg * 1e6)
-            ach, frac = f"{rate:.1f} TFLOP/s", f"{100 * rate / MFMA_FP32_PEAK_TFLOPS:.1f} %"
+            ach, frac = f"{rate:.1f} TFLOP/s", f"{100 * rate / (MFMA_BF16_PARTS_PEAK_TFLOPS if e['parts'] else MFMA_FP32_PEAK_TFLOPS):.1f} %"
         elif e["bytes"]:
             alg = f"{e['bytes'] / 1e6:.1f} MB"
             rate = e["bytes"] / (avg * 1e3)
@@ -105,9 +106,8 @@ def summarize(a) -> str:
         if mfma:
             m = mfma.get(k, {})
             util = m.get("MfmaUtil")
-            fl = m.get("MfmaFlopsF32")
-            line += (f" {util:.1f} % |" if util is not None else " – |") + \
-                    (f" {fl / e['flops']:.4f} |" if fl is not None and e["flops"] else " – |") + \
+            per_flop = [f" {m[c] / e['flops']:.4f} |" if c in m and e["flops"] else " – |" for c in ("MfmaFlopsF32", "MfmaFlopsBF16")]
+            line += (f" {util:.1f} % |" if util is not None else " – |") + "".join(per_flop) + \
                     (f" {m['LDSBankConflict']:.1f} % |" if "LDSBankConflict" in m else " – |")
         out.append(line)
     if a.events:
