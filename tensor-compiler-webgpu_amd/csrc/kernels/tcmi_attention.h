@@ -22,7 +22,8 @@
 //           part g are exactly the MFMA's A operand for k = 16g + 4q + s, so P
 //           goes from the score registers into the second product directly.
 // Both products walk their k index 16 at a time, s inner (the order of
-// tcmi_gemm.h), so the scores equal a tcmi_gemm.h product's bit for bit.
+// tcmi_gemm.h), so the scores equal a tcmi_gemm.h product's bit for bit (heads of 96 and more: the
+// separate product may be one in bf16 parts, equal within the float32 budget).
 
 #pragma once
 

@@ -43,10 +43,11 @@
 // barrier of a slice stands before its last column, which multiplies while the next
 // slice's first fragments are read.
 //
-// What bounds it: power, then LDS. 4096^3 takes 620 us (222 TFLOP/s; the fp32 kernel 1040 us,
-// 132): MFMAs alone on such values run at 1.9 PFLOP/s, 310 of these, as the clock drops to
-// about 1.95 GHz, and the same launch on zeros takes 547 us. The 64-wide tiles move 1.5 times the
-// LDS bytes per flop and are bound by them (128 bytes a cycle a CU). Tried: 128 x 256 tiles
+// What bounds it: power, where tiles are many. 4096^3 takes 610 - 640 us (220 TFLOP/s; the fp32 kernel
+// 1040 us, 132) in 1.33 M cycles, the matrix cores busy for 59 % of them and LDS for 26 %, at 2.07 GHz; on
+// zeros the same cycles run at 2.39 GHz, 543 us. With one tile a CU (8192 x 1024 x 256, 39 us at 2.4 GHz)
+// the matrix cores are busy for 26 % and LDS for 23 %: the chain of a slice from its loads to its
+// products stands open. Tried: 128 x 256 tiles
 // by 4 wavefronts of 64 x 128 (less LDS traffic, one wavefront per SIMD) 707 us; two or four
 // slices of loads in flight, and K groups inside a workgroup, no faster.
 
