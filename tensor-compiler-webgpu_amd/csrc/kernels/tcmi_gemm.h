@@ -214,6 +214,8 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
   };
   Stage st0, st1;
 
+  // The three conditions of a load are one mask (&, not &&): as nested branches, a 64 x 64 tile's
+  // split product (64 x 3328 x 64) took 11.6 us instead of 10.3.
   auto load_slice = [&](Stage& S, uint32_t k0) {
     float4* ra = S.ra;
     float4* rb = S.rb;
@@ -225,7 +227,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const int t = tid + v * THREADS;
         const uint32_t row = t / (BK / 4), kk = (t % (BK / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (t < BM * BK / 4 && m0 + row < M && k0 + kk < kend) {
+        if ((t < BM * BK / 4) & (m0 + row < M) & (k0 + kk < kend)) {
           if constexpr (view_run<AV>(0) != 0) x = load_run4(Ab + vrow<AV>(m0 + row) + vcol<AV>(k0 + kk), run_over(k0 + kk, kend));
           else x = *reinterpret_cast<const float4*>(Ab + vrow<AV>(m0 + row) + vcol<AV>(k0 + kk));
         }
@@ -237,7 +239,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const int t = tid + v * THREADS;
         const uint32_t kk = t / (BM / 4), row = (t % (BM / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (t < BM * BK / 4 && m0 + row < M && k0 + kk < kend) {
+        if ((t < BM * BK / 4) & (m0 + row < M) & (k0 + kk < kend)) {
           if constexpr (view_run<AV>(0) != 0) x = load_run4(Ab + vcol<AV>(k0 + kk) + vrow<AV>(m0 + row), run_over(m0 + row, M));
           else x = *reinterpret_cast<const float4*>(Ab + vcol<AV>(k0 + kk) + vrow<AV>(m0 + row));
         }
@@ -249,7 +251,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const int t = tid + v * THREADS;
         const uint32_t row = t / BK, kk = t % BK;
         float x = 0.f;
-        if (t < BM * BK && m0 + row < M && k0 + kk < kend) x = Ab[vrow<AV>(m0 + row) + vcol<AV>(k0 + kk)];
+        if ((t < BM * BK) & (m0 + row < M) & (k0 + kk < kend)) x = Ab[vrow<AV>(m0 + row) + vcol<AV>(k0 + kk)];
         sa[v] = x;
       }
     }
@@ -259,7 +261,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const int t = tid + v * THREADS;
         const uint32_t kk = t / (BN / 4), c = (t % (BN / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (t < BK * BN / 4 && k0 + kk < kend && n0 + c < N) {
+        if ((t < BK * BN / 4) & (k0 + kk < kend) & (n0 + c < N)) {
           if constexpr (view_run<BV>(0) != 0) x = load_run4(Bb + vrow<BV>(k0 + kk) + vcol<BV>(n0 + c), run_over(n0 + c, N));
           else x = *reinterpret_cast<const float4*>(Bb + vrow<BV>(k0 + kk) + vcol<BV>(n0 + c));
         }
@@ -271,7 +273,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const int t = tid + v * THREADS;
         const uint32_t c = t / (BK / 4), kk = (t % (BK / 4)) * 4;
         float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (t < BK * BN / 4 && k0 + kk < kend && n0 + c < N) {
+        if ((t < BK * BN / 4) & (k0 + kk < kend) & (n0 + c < N)) {
           if constexpr (view_run<BV>(0) != 0) x = load_run4(Bb + vcol<BV>(n0 + c) + vrow<BV>(k0 + kk), run_over(k0 + kk, kend));
           else x = *reinterpret_cast<const float4*>(Bb + vcol<BV>(n0 + c) + vrow<BV>(k0 + kk));
         }
@@ -283,7 +285,7 @@ __device__ __forceinline__ void gemm_f32_sum(float* const As_, float* const Bs_,
         const int t = tid + v * THREADS;
         const uint32_t kk = t / BN, c = t % BN;
         float x = 0.f;
-        if (t < BK * BN && k0 + kk < kend && n0 + c < N) x = Bb[vrow<BV>(k0 + kk) + vcol<BV>(n0 + c)];
+        if ((t < BK * BN) & (k0 + kk < kend) & (n0 + c < N)) x = Bb[vrow<BV>(k0 + kk) + vcol<BV>(n0 + c)];
         sb[v] = x;
       }
     }
